@@ -343,9 +343,10 @@ struct DbDev {
         ptable.release(); ptable_host.clear();
         paged = false; page_elems = npages = nslot = rot = nfixed_used = 0; host_u = nullptr;
     }
-    DBuf<float> mp_s, mp_z;
+    DBuf<float4> cell_mp;
+    DBuf<uint8_t> cell_ring;
     DBuf<double> econ, ejac;
-    DBuf<int> eltype, axis, cell_start, cell_elems;
+    DBuf<int> eltype, axis, cell_start;
     std::vector<double> econ_host;
     std::vector<int> eltype_host, axis_host;
     int nvar = 0;
@@ -493,8 +494,21 @@ int upload_db(DbDev &D, const mck_db_t &db, int nt, const char *name, int page_e
         smin = std::min(smin, db.mp_s[e]); smax = std::max(smax, db.mp_s[e]);
         zmin = std::min(zmin, db.mp_z[e]); zmax = std::max(zmax, db.mp_z[e]);
     }
-    double area = std::max(1.0, (double)(smax - smin)) * std::max(1.0, (double)(zmax - zmin));
-    double h = std::sqrt(area * 2.0 / ne);
+    // cells as large as the element that 80 % of the elements do not exceed (element sizes
+    // grow with the radius: cells by the mean area left most cells of the mantle empty), at
+    // most 4 cells per element
+    double h = 0.0;
+    {
+        std::vector<double> ea(ne);
+        for (int e = 0; e < ne; ++e) {
+            const double *E = &D.econ_host[(size_t)e * 16];
+            ea[e] = 0.5 * std::fabs((E[2] - E[0]) * (E[7] - E[5]) - (E[3] - E[1]) * (E[6] - E[4]));
+        }
+        const int at = (int)(0.8 * (ne - 1));
+        std::nth_element(ea.begin(), ea.begin() + at, ea.end());
+        const double area = std::max(1.0, (double)(smax - smin)) * std::max(1.0, (double)(zmax - zmin));
+        h = std::sqrt(std::max(ea[at], area / (4.0 * ne)));
+    }
     int gnx = std::max(1, (int)std::ceil((smax - smin) / h) + 1);
     int gnz = std::max(1, (int)std::ceil((zmax - zmin) / h) + 1);
     std::vector<int> cnt((size_t)gnx * gnz + 1, 0), cell(ne);
@@ -505,22 +519,49 @@ int upload_db(DbDev &D, const mck_db_t &db, int nt, const char *name, int page_e
         cnt[cell[e] + 1]++;
     }
     for (size_t i = 1; i < cnt.size(); ++i) cnt[i] += cnt[i - 1];
-    std::vector<int> elems(ne), fill(cnt.begin(), cnt.end() - 1);
-    for (int e = 0; e < ne; ++e) elems[fill[cell[e]]++] = e;
-    HIPCHECK(D.mp_s.ensure(ne));
-    HIPCHECK(D.mp_z.ensure(ne));
+    std::vector<float4> elems(ne);
+    std::vector<int> fill(cnt.begin(), cnt.end() - 1);
+    for (int e = 0; e < ne; ++e) {
+        float id;
+        std::memcpy(&id, &e, 4);
+        elems[fill[cell[e]]++] = make_float4(db.mp_s[e], db.mp_z[e], id, 0.0f);
+    }
+    // rings around every cell whose block of cells holds kFirstBlock midpoints (or all)
+    std::vector<uint8_t> ring((size_t)gnx * gnz);
+    {
+        const int w = gnx + 1;
+        std::vector<int> sum((size_t)w * (gnz + 1), 0);         // midpoints of the cells [0, iz) x [0, ix)
+        for (int iz = 0; iz < gnz; ++iz)
+            for (int ix = 0; ix < gnx; ++ix) {
+                const int c = iz * gnx + ix;
+                sum[(size_t)(iz + 1) * w + ix + 1] = cnt[c + 1] - cnt[c] + sum[(size_t)iz * w + ix + 1]
+                                                   + sum[(size_t)(iz + 1) * w + ix] - sum[(size_t)iz * w + ix];
+            }
+        for (int iz = 0; iz < gnz; ++iz)
+            for (int ix = 0; ix < gnx; ++ix) {
+                int r = 1;
+                for (; r < 255; ++r) {
+                    const int a = std::max(0, ix - r), b = std::min(gnx, ix + r + 1);
+                    const int c = std::max(0, iz - r), d = std::min(gnz, iz + r + 1);
+                    const int n = sum[(size_t)d * w + b] - sum[(size_t)c * w + b] - sum[(size_t)d * w + a]
+                                + sum[(size_t)c * w + a];
+                    if (n >= std::min(kFirstBlock, ne)) break;
+                }
+                ring[(size_t)iz * gnx + ix] = (uint8_t)r;
+            }
+    }
+    HIPCHECK(D.cell_ring.ensure(ring.size()));
+    HIPCHECK(D.cell_mp.ensure(ne));
     HIPCHECK(D.econ.ensure((size_t)ne * 16));
     HIPCHECK(D.eltype.ensure(ne));
     HIPCHECK(D.axis.ensure(ne));
     HIPCHECK(D.cell_start.ensure(cnt.size()));
-    HIPCHECK(D.cell_elems.ensure(ne));
-    HIPCHECK(hipMemcpy(D.mp_s.p, db.mp_s, ne * 4, hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(D.mp_z.p, db.mp_z, ne * 4, hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(D.econ.p, D.econ_host.data(), (size_t)ne * 16 * 8, hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(D.eltype.p, db.eltype, ne * 4, hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(D.axis.p, db.axis, ne * 4, hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(D.cell_start.p, cnt.data(), cnt.size() * 4, hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(D.cell_elems.p, elems.data(), ne * 4, hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(D.cell_mp.p, elems.data(), ne * sizeof(float4), hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(D.cell_ring.p, ring.data(), ring.size(), hipMemcpyHostToDevice));
     // snapshots: use in place when they already live in device memory, page them from
     // host memory when asked to, else copy them once
     D.elem_floats = (size_t)db.nvar * 25 * nt;
@@ -564,10 +605,9 @@ int upload_db(DbDev &D, const mck_db_t &db, int nt, const char *name, int page_e
     D.d.u = u;
     D.d.u_first = 0;
     D.d.u_last = D.paged ? std::min(ne, D.page_elems) : ne;
-    D.d.mp_s = D.mp_s.p; D.d.mp_z = D.mp_z.p;
     D.d.econ = D.econ.p; D.d.eltype = D.eltype.p; D.d.axis = D.axis.p;
     D.d.gnx = gnx; D.d.gnz = gnz; D.d.gs0 = smin; D.d.gz0 = zmin; D.d.gh = h;
-    D.d.cell_start = D.cell_start.p; D.d.cell_elems = D.cell_elems.p;
+    D.d.cell_start = D.cell_start.p; D.d.cell_mp = D.cell_mp.p; D.d.cell_ring = D.cell_ring.p;
     D.d.amplitude = db.amplitude;
     return MCK_OK;
 }
@@ -958,6 +998,16 @@ int spt_for(int nt) {
 }
 
 unsigned grid_x8(int n) { return 8u * (unsigned)((n + 7) / 8); }
+
+// points xyz[npts] located in the frames frame0 .. frame0 + nframes - 1 (mesh of D): out
+// [npts][nframes]; active (nullable): receivers in use of each voxel (P points)
+hipError_t launch_locate(State &G, const DbDev &D, int frame0, int nframes, int npts, const double *xyz,
+                         const uint8_t *active, int P, Located *out) {
+    const long long lanes = (long long)npts * nframes * kLocLanes;
+    hipLaunchKernelGGL(k_locate, dim3((unsigned)((lanes + 63) / 64)), dim3(64), 0, G.stream, D.d, G.frames.p, frame0,
+                       nframes, npts, xyz, G.S.planet_radius, active, P, G.R, out, G.err.p);
+    return hipGetLastError();
+}
 
 // operator set-up of n points (fwd) or pairs (bwd) in launch order (null = identity)
 hipError_t launch_setup(State &G, bool fwd, int n, const int *order, const int *keys, const Located *loc) {
@@ -1398,9 +1448,7 @@ int reciprocity_seismograms(State &G) {
     if (e == hipSuccess) e = hipMemcpy(d_xyz, G.src_r, 3 * sizeof(double), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemsetAsync(G.err.p, 0, 4, G.stream);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_locate, dim3((R + 127) / 128), dim3(128), 0, G.stream, G.fwd.d, G.frames.p, 1, R, 1,
-                           d_xyz, S.planet_radius, nullptr, 1, R, d_loc, G.err.p);
-        e = hipGetLastError();
+        e = launch_locate(G, G.fwd, 1, R, 1, d_xyz, nullptr, 1, d_loc);
     }
     if (e == hipSuccess) e = hipMemcpyAsync(loc.data(), d_loc, (size_t)R * sizeof(Located), hipMemcpyDeviceToHost, G.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(G.stream);
@@ -1976,12 +2024,8 @@ int eval_chunk(State &G, int P, int w0, int nw, std::vector<std::pair<hipEvent_t
                        tet_basis ? G.bweights.p + (size_t)w0 * P * 4 : nullptr, G.err.p);
     HIPCHECK(hipGetLastError());
     // fwd and bwd meshes may differ: locate frame 0 in the fwd mesh, frames 1.. in the bwd mesh
-    hipLaunchKernelGGL(k_locate, dim3((unsigned)((np + 127) / 128)), dim3(128), 0, st, G.fwd.d,
-                       G.frames.p, 0, 1, np, G.xyz.p, G.S.planet_radius, nullptr, P, R, loc_f, G.err.p);
-    HIPCHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_locate, dim3((unsigned)(((long long)np * R + 127) / 128)), dim3(128), 0, st,
-                       G.bwd.d, G.frames.p, 1, R, np, G.xyz.p, G.S.planet_radius, act, P, R, loc_b, G.err.p);
-    HIPCHECK(hipGetLastError());
+    HIPCHECK(launch_locate(G, G.fwd, 0, 1, np, G.xyz.p, nullptr, P, loc_f));
+    HIPCHECK(launch_locate(G, G.bwd, 1, R, np, G.xyz.p, act, P, loc_b));
     hipLaunchKernelGGL(k_count_points, dim3((nw + 255) / 256), dim3(256), 0, st, nw, R, P, act,
                        G.elem_count.p + 4);
     HIPCHECK(hipGetLastError());
@@ -2286,9 +2330,7 @@ int points_upload(State &G, int npts, const double *xyz) {
 int locate_frame(State &G, int frame, int npts) {
     const DbDev &D = frame == 0 ? G.fwd : G.bwd;
     // results for frame f of point p at loc[p] (stride 1)
-    hipLaunchKernelGGL(k_locate, dim3((npts + 127) / 128), dim3(128), 0, G.stream, D.d, G.frames.p, frame,
-                       1, npts, G.xyz.p, G.S.planet_radius, nullptr, 1, G.R, G.loc.p, G.err.p);
-    HIPCHECK(hipGetLastError());
+    HIPCHECK(launch_locate(G, D, frame, 1, npts, G.xyz.p, nullptr, 1, G.loc.p));
     return MCK_OK;
 }
 
@@ -2729,11 +2771,8 @@ int mck_base_kernels(int32_t npts, const double *xyz, double *base) {
     }
     HIPCHECK(hipMemcpyAsync(G.model_idx.p, midx.data(), npts * 4, hipMemcpyHostToDevice, G.stream));
     Located *loc_f = G.loc.p, *loc_b = G.loc.p + npts;
-    hipLaunchKernelGGL(k_locate, dim3((npts + 127) / 128), dim3(128), 0, G.stream, G.fwd.d, G.frames.p, 0, 1,
-                       npts, G.xyz.p, G.S.planet_radius, nullptr, 1, R, loc_f, G.err.p);
-    hipLaunchKernelGGL(k_locate, dim3(((long long)npts * R + 127) / 128), dim3(128), 0, G.stream, G.bwd.d,
-                       G.frames.p, 1, R, npts, G.xyz.p, G.S.planet_radius, nullptr, 1, R, loc_b, G.err.p);
-    HIPCHECK(hipGetLastError());
+    HIPCHECK(launch_locate(G, G.fwd, 0, 1, npts, G.xyz.p, nullptr, 1, loc_f));
+    HIPCHECK(launch_locate(G, G.bwd, 1, R, npts, G.xyz.p, nullptr, 1, loc_b));
     double *d_base = nullptr, *d_phys = nullptr;
     HIPCHECK(hipMalloc((void **)&d_base, (size_t)npts * G.nk * 6 * 8));
     if (hipMalloc((void **)&d_phys, (size_t)npts * G.nk * 8) != hipSuccess) {
@@ -3336,8 +3375,8 @@ void mck_finalize(void) {
         if (D->u_owned) (void)hipFree(D->u_owned);
         D->u_owned = nullptr;
         D->release_pages();
-        D->mp_s.release(); D->mp_z.release(); D->econ.release(); D->ejac.release(); D->eltype.release();
-        D->axis.release(); D->cell_start.release(); D->cell_elems.release();
+        D->econ.release(); D->ejac.release(); D->eltype.release();
+        D->axis.release(); D->cell_start.release(); D->cell_mp.release(); D->cell_ring.release();
     }
     G.frames.release(); G.twq.release(); G.twq_d.release(); G.H.release(); G.recs.release();
     G.recs_base.release(); G.kerns_base.release();

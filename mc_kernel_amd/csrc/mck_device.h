@@ -9,6 +9,7 @@ namespace mck {
 constexpr int kMaxSim = 4;       // fwd simulations MZZ, MXX+MYY, MXZ, MXY
 constexpr int kMaxVar = 10;      // merged variables per element (fwd)
 constexpr int kMaxKernelsPerRec = 256;
+constexpr int kFirstBlock = 28;  // midpoints of a query's first block of grid cells
 constexpr int kNN = 12;          // nearest midpoints tested (readfields.f90:1067)
 constexpr int kStrainThreads = 256;
 constexpr int kEvalThreads = 256;
@@ -45,7 +46,6 @@ struct DevDb {
     // each page (null: not held), page_elems elements each; u is then unused
     const float *const *page_u;
     int page_elems;
-    const float *mp_s, *mp_z; // element midpoints
     const double *econ;       // [nelem][16] element constants (see host setup)
     const double *ejac;       // [nelem][25][5] inverse Jacobian and 1/s at the nodes
     const int *eltype, *axis;
@@ -53,7 +53,8 @@ struct DevDb {
     int gnx, gnz;
     double gs0, gz0, gh;      // origin and cell size (m)
     const int *cell_start;    // [gnx*gnz+1]
-    const int *cell_elems;    // element ids sorted by cell
+    const float4 *cell_mp;    // midpoints sorted by cell: s, z, element id (bits), unused
+    const uint8_t *cell_ring; // rings around the cell whose block holds kFirstBlock midpoints
     double amplitude;
 };
 

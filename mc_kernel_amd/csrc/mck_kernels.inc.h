@@ -143,28 +143,6 @@ __device__ inline void d_inv_jacobian(double xi, double eta, const double *E, in
     ij[3] = J0 / det;
 }
 
-// inv_mapping_* + inside_element (finite_elem_mapping.f90:101-141, 137-200, 403-433,
-// 505-535): 10 Newton steps from the centre; single-precision threshold 1e-7**2 except
-// for spheroids (1d-7**2).
-__device__ inline bool d_inside(double s, double z, const double *E, int type, double *xi_out,
-                                double *eta_out)
-{
-    const double thr = (type == 0) ? (1e-7 * 1e-7) : (double)(1e-7f * 1e-7f);
-    double xi = 0.0, eta = 0.0, sz[2], ij[4];
-    for (int i = 1; i <= 10; ++i) {
-        d_mapping(xi, eta, E, type, sz);
-        double ds = s - sz[0], dz = z - sz[1];
-        if ((ds * ds + dz * dz) / (s * s + z * z) < thr) break;
-        d_inv_jacobian(xi, eta, E, type, ij);
-        xi = xi + ij[0] * ds + ij[2] * dz;
-        eta = eta + ij[1] * ds + ij[3] * dz;
-    }
-    *xi_out = xi;
-    *eta_out = eta;
-    const double tol = 1e-3;
-    return (xi >= -1 - tol && xi <= 1 + tol && eta >= -1 - tol && eta <= 1 + tol);
-}
-
 // gfortran NORM2 of a 3-vector (scaled sum of squares)
 __device__ inline double d_norm2(double a, double b, double c)
 {
@@ -594,34 +572,115 @@ __global__ __launch_bounds__(64) void k_hetero_integral(int nelem, const double 
 }
 
 // ------------------------------------------------------------------------------------
-// k_locate: one thread per (point, frame).  Frame 0 = source, 1 + r = receiver r.
+// k_locate: kLocLanes lanes per (point, frame).  Frame 0 = source, 1 + r = receiver r.
 // active (nullable) gates bwd frames: active[slot_of_point * R + r].
+//
+// The lanes of a query read the midpoints of a block of grid cells together (a row of
+// cells per lane; the block's size comes with the cell, so that it holds about twice the
+// 13 nearest), keep the 13 nearest as sorted 64-bit keys (fp32 distance bits, element id)
+// spread over the lanes, and run the Newton inversions of the nearest 8 candidates at
+// once, stopping when the first of them in distance order that holds the point is known.
+// What bounds it: a serial chain of FP64 operations and dependent loads (latency at small
+// launches, FP64 issue at large ones).  One thread per query with the sorted list in
+// scratch memory and a search by single rings of cells took 260 us for a launch of 96
+// points and 0.79 ms for 62,000 points x 10 receivers (12,000 voxels of c1); 8 lanes take
+// 20 us and 0.51 ms.  (The Newton loop is not unrolled and the function is inlined: the
+// unrolled form, called, exceeds the range of a branch.)
 // ------------------------------------------------------------------------------------
-__device__ inline void knn_insert(float d, int e, float *bd, int *bi, int &cnt)
+constexpr int kLocLanes = 8;
+constexpr int kLocSlots = 8;                  // keys per lane: 2 of the kept 13, 6 new ones
+constexpr unsigned long long kNoKey = ~0ull;
+
+// the other lane's key, by DPP (CTRL: a permutation inside the query's 8 lanes)
+template <int CTRL>
+__device__ __forceinline__ unsigned long long dpp_key(unsigned long long k)
 {
-    const int K = kNN + 1;
-    if (cnt == K && !(d < bd[K - 1] || (d == bd[K - 1] && e < bi[K - 1]))) return;
-    int p = (cnt < K) ? cnt++ : K - 1;
-    while (p > 0 && (bd[p - 1] > d || (bd[p - 1] == d && bi[p - 1] > e))) {
-        bd[p] = bd[p - 1];
-        bi[p] = bi[p - 1];
-        --p;
-    }
-    bd[p] = d;
-    bi[p] = e;
+    const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)k, CTRL, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(k >> 32), CTRL, 0xF, 0xF, true);
+    return ((unsigned long long)hi << 32) | lo;
 }
 
-__global__ void k_locate(DevDb db, const DevFrame *frames, int frame0, int nframes, int npts,
-                         const double *xyz, double planet_radius, const uint8_t *active,
-                         int P, int R, Located *out, int *err)
+// smallest key of the query's 8 lanes, in every lane
+__device__ __forceinline__ unsigned long long loc_min8(unsigned long long k)
 {
-    int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= npts * nframes) return;
-    int p = gid / nframes, f = frame0 + (gid - (gid / nframes) * nframes);
+    unsigned long long o = dpp_key<0xB1>(k);      // lanes 1 0 3 2
+    k = o < k ? o : k;
+    o = dpp_key<0x4E>(k);                         // lanes 2 3 0 1
+    k = o < k ? o : k;
+    o = dpp_key<0x141>(k);                        // lanes 7 6 5 4 3 2 1 0
+    return o < k ? o : k;
+}
+
+// bits of the query's 8 lanes in a wave vote
+__device__ __forceinline__ unsigned loc_vote(bool c)
+{
+    return (unsigned)(__ballot(c) >> (__lane_id() & ~(kLocLanes - 1u))) & ((1u << kLocLanes) - 1u);
+}
+
+__device__ __forceinline__ void loc_order(unsigned long long &a, unsigned long long &b)
+{
+    const bool sw = b < a;
+    const unsigned long long t = sw ? b : a;
+    b = sw ? a : b;
+    a = t;
+}
+
+// inv_mapping_* + inside_element (finite_elem_mapping.f90:101-141, 137-200, 403-433,
+// 505-535) of this lane's candidate e (-1: none): at most 10 Newton steps from the centre;
+// single-precision threshold 1e-7**2 except for spheroids (1d-7**2).  The query's lanes go
+// in step: returns the first lane (in lane order) whose candidate holds the point, or -1,
+// as soon as that lane and all before it have finished.
+__device__ __forceinline__ int loc_inside(double s, double z, const DevDb &db, int e, double &xi, double &eta)
+{
+    const double tol = 1e-3;
+    const int type = e >= 0 ? db.eltype[e] : 1;
+    const double *Eg = db.econ + (size_t)max(e, 0) * 16;
+    double E[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) E[i] = Eg[i];
+    const double thr = (type == 0) ? (1e-7 * 1e-7) : (double)(1e-7f * 1e-7f);
+    bool fin = e < 0;
+    xi = 0.0;
+    eta = 0.0;
+#pragma unroll 1
+    for (int i = 1; i <= 10; ++i) {
+        if (!fin) {
+            double sz[2], ij[4];
+            d_mapping(xi, eta, E, type, sz);
+            const double ds = s - sz[0], dz = z - sz[1];
+            if ((ds * ds + dz * dz) / (s * s + z * z) < thr) {
+                fin = true;
+            } else {
+                d_inv_jacobian(xi, eta, E, type, ij);
+                xi = xi + ij[0] * ds + ij[2] * dz;
+                eta = eta + ij[1] * ds + ij[3] * dz;
+            }
+        }
+        if (i == 10) fin = true;
+        const bool in = e >= 0 && fin && xi >= -1 - tol && xi <= 1 + tol && eta >= -1 - tol && eta <= 1 + tol;
+        const unsigned vf = loc_vote(fin), vi = loc_vote(in);
+        if (vi) {
+            const int f = __ffs((int)vi) - 1;
+            if ((vf & ((1u << f) - 1u)) == (1u << f) - 1u) return f;
+        } else if (vf == (1u << kLocLanes) - 1u) {
+            return -1;
+        }
+    }
+    return -1;
+}
+
+__global__ __launch_bounds__(64) void k_locate(DevDb db, const DevFrame *frames, int frame0, int nframes, int npts,
+                                               const double *xyz, double planet_radius, const uint8_t *active,
+                                               int P, int R, Located *out, int *err)
+{
+    const long long gid = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kLocLanes;
+    const int sub = threadIdx.x & (kLocLanes - 1);
+    if (gid >= (long long)npts * nframes) return;
+    const int p = (int)(gid / nframes), f = frame0 + (int)(gid - (long long)p * nframes);
     Located res;
     res.elem = -1; res.tie = 0; res.xi = 0; res.eta = 0; res.phi = 0;
     if (f > 0 && active && !active[(p / P) * R + (f - 1)]) {
-        out[gid] = res;
+        if (sub == 0) out[gid] = res;
         return;
     }
     const DevFrame fr = frames[f];
@@ -638,53 +697,109 @@ __global__ void k_locate(DevDb db, const DevFrame *frames, int frame0, int nfram
     res.phi = (pc < 0.0) ? 2.0 * 3.1415926535898 + pc : pc;
     double d2 = s * s + z * z, Rp = planet_radius;
     if (d2 > Rp * Rp) { s = s / sqrt(d2) * Rp; z = z / sqrt(d2) * Rp; }
-    // exact 13 nearest midpoints (12 tested, the 13th detects ties at the boundary)
-    float qs = (float)s, qz = (float)z;
-    float bd[kNN + 1];
-    int bi[kNN + 1], cnt = 0;
+    // exact 13 nearest midpoints (12 tested, the 13th detects ties at the boundary) by
+    // (fp32 distance, element): keys k[0] (ranks 0 .. 7, one per lane) and k[1] (8 .. 12)
+    const float qs = (float)s, qz = (float)z;
+    unsigned long long k[kLocSlots], bound = kNoKey;           // bound: the 13th key
+    k[0] = k[1] = kNoKey;
     int cx = (int)floor((s - db.gs0) / db.gh), cz = (int)floor((z - db.gz0) / db.gh);
     cx = cx < 0 ? 0 : (cx >= db.gnx ? db.gnx - 1 : cx);
     cz = cz < 0 ? 0 : (cz >= db.gnz ? db.gnz - 1 : cz);
-    for (int ring = 0;; ++ring) {
-        int x0 = cx - ring, x1 = cx + ring, z0 = cz - ring, z1 = cz + ring;
-        for (int iz = z0; iz <= z1; ++iz) {
-            if (iz < 0 || iz >= db.gnz) continue;
-            bool edge_z = (iz == z0 || iz == z1);
-            for (int ix = x0; ix <= x1; ++ix) {
-                if (ix < 0 || ix >= db.gnx) continue;
-                if (!edge_z && ix != x0 && ix != x1) continue;
-                int c = iz * db.gnx + ix;
-                for (int k = db.cell_start[c]; k < db.cell_start[c + 1]; ++k) {
-                    int e = db.cell_elems[k];
-                    float dx = db.mp_s[e] - qs, dz = db.mp_z[e] - qz;
+    const int first_ring = db.cell_ring[cz * db.gnx + cx];
+    for (int ring = first_ring;; ++ring) {
+        // the block of rings 0 .. first_ring row by row, then one ring after another: its
+        // first and last rows whole, the cells at both ends of the others.  Lane i takes
+        // the rows i, i + 8, ..; a row's cells lie next to each other in cell_mp.
+        const int x0 = cx - ring, x1 = cx + ring, z0 = cz - ring, z1 = cz + ring;
+        int iz = z0 + sub, right = 0, pos = 0, end = 0;
+        for (;;) {
+            while (pos >= end && iz <= z1) {
+                const bool ends = ring > first_ring && iz != z0 && iz != z1;
+                const int xa = max(ends && right ? x1 : x0, 0), xb = min(ends && !right ? x0 : x1, db.gnx - 1);
+                if (iz >= 0 && iz < db.gnz && xa <= xb) {
+                    const int *row = db.cell_start + iz * db.gnx;
+                    pos = row[xa];
+                    end = row[xb + 1];
+                }
+                if (ends && !right) right = 1;
+                else { iz += kLocLanes; right = 0; }
+            }
+            // (all slots are free at first: no key kept yet)
+            const int kept = bound == kNoKey && k[0] == kNoKey ? 0 : 2;
+            bool some = false;
+#pragma unroll
+            for (int q = 0; q < kLocSlots; ++q) {
+                unsigned long long key = kNoKey;
+                if (q >= kept && pos + (q - kept) < end) {
+                    const float4 c = db.cell_mp[pos + (q - kept)];
+                    const float dx = c.x - qs, dz = c.y - qz;
                     float sd = 0.0f;
                     sd = sd + dx * dx;
                     sd = sd + dz * dz;
-                    knn_insert(sd, e, bd, bi, cnt);
+                    key = ((unsigned long long)__float_as_uint(sd) << 32) | (unsigned)__float_as_int(c.z);
+                }
+                if (q >= kept) {
+                    k[q] = key < bound ? key : kNoKey;
+                    some |= k[q] != kNoKey;
                 }
             }
+            pos = min(pos + kLocSlots - kept, end);
+            if (loc_vote(some)) {
+                // this lane's keys in order (a sorting network of 8), then the 13 smallest of the
+                // query, rank by rank
+                loc_order(k[0], k[1]); loc_order(k[2], k[3]); loc_order(k[4], k[5]); loc_order(k[6], k[7]);
+                loc_order(k[0], k[2]); loc_order(k[1], k[3]); loc_order(k[4], k[6]); loc_order(k[5], k[7]);
+                loc_order(k[1], k[2]); loc_order(k[5], k[6]); loc_order(k[0], k[4]); loc_order(k[3], k[7]);
+                loc_order(k[1], k[5]); loc_order(k[2], k[6]);
+                loc_order(k[1], k[4]); loc_order(k[3], k[6]);
+                loc_order(k[2], k[4]); loc_order(k[3], k[5]);
+                loc_order(k[3], k[4]);
+                unsigned long long n0 = kNoKey, n1 = kNoKey, prev = kNoKey;
+                int tie = 0;
+#pragma unroll
+                for (int j = 0; j <= kNN; ++j) {
+                    const unsigned long long m = loc_min8(k[0]);
+                    if (m == k[0]) {
+#pragma unroll
+                        for (int q = 0; q + 1 < kLocSlots; ++q) k[q] = k[q + 1];
+                        k[kLocSlots - 1] = kNoKey;
+                    }
+                    if (sub == (j & (kLocLanes - 1))) {
+                        if (j < kLocLanes) n0 = m; else n1 = m;
+                    }
+                    if (m != kNoKey && prev != kNoKey && (unsigned)(m >> 32) == (unsigned)(prev >> 32)) tie = 1;
+                    prev = m;
+                }
+                bound = prev;
+                res.tie = tie;
+                k[0] = n0;
+                k[1] = n1;
+            }
+            if (!loc_vote(pos < end || iz <= z1)) break;
         }
-        bool all = (x0 <= 0 && z0 <= 0 && x1 >= db.gnx - 1 && z1 >= db.gnz - 1);
-        if (all) break;
-        if (cnt == kNN + 1) {
+        if (x0 <= 0 && z0 <= 0 && x1 >= db.gnx - 1 && z1 >= db.gnz - 1) break;
+        if (bound != kNoKey) {
             double inf = 1e300;
             double lo_s = x0 <= 0 ? -inf : db.gs0 + x0 * db.gh, hi_s = x1 >= db.gnx - 1 ? inf : db.gs0 + (x1 + 1) * db.gh;
             double lo_z = z0 <= 0 ? -inf : db.gz0 + z0 * db.gh, hi_z = z1 >= db.gnz - 1 ? inf : db.gz0 + (z1 + 1) * db.gh;
             double dm = fmin(fmin((double)qs - lo_s, hi_s - (double)qs), fmin((double)qz - lo_z, hi_z - (double)qz));
-            if (dm > 0 && (double)bd[kNN] < dm * dm * (1.0 - 1e-6)) break;
+            if (dm > 0 && (double)__uint_as_float((unsigned)(bound >> 32)) < dm * dm * (1.0 - 1e-6)) break;
         }
     }
-    for (int j = 1; j < cnt; ++j) if (bd[j] == bd[j - 1]) res.tie = 1;
-    for (int c = 0; c < kNN && c < cnt; ++c) {
-        int e = bi[c];
-        double xi, eta;
-        if (d_inside(s, z, db.econ + (size_t)e * 16, db.eltype[e], &xi, &eta)) {
-            res.elem = e; res.xi = xi; res.eta = eta;
-            break;
-        }
+    // the first of the 12 nearest that holds the point: the nearest 8, then the other 4
+    double xi = 0.0, eta = 0.0;
+    int e = -1, first = -1;
+#pragma unroll 1
+    for (int half = 0; half < 2 && first < 0; ++half) {
+        const unsigned long long key = half == 0 ? k[0] : (sub < kNN - kLocLanes ? k[1] : kNoKey);
+        e = key != kNoKey ? (int)(unsigned)key : -1;
+        first = loc_inside(s, z, db, e, xi, eta);
     }
-    if (res.elem < 0 && err) atomicOr(err, 1);
-    out[gid] = res;
+    if (sub == max(first, 0)) {
+        if (first >= 0) { res.elem = e; res.xi = xi; res.eta = eta; }
+        else if (err) atomicOr(err, 1);
+        out[gid] = res;
+    }
 }
 
 // ------------------------------------------------------------------------------------
