@@ -1174,7 +1174,6 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
     const size_t per_elem = (size_t)J * pc.ustride * sizeof(float2);
     const int batch = (int)std::max<size_t>(1, std::min<size_t>((size_t)nerun, G.uspec_budget / per_elem));
     HIPCHECK(G.Uspec.ensure((size_t)batch * J * pc.ustride));
-    const size_t smem_s = 2 * (size_t)pc.M * sizeof(double2);
     const size_t smem_m = mfma_wave_lds(KS, pc.nd_b, pc.max_cls);
     const int spt = spt_for(pc.nt);
     G.stats.spt = spt;
@@ -1186,10 +1185,13 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
         bool launched = false;
 #define SPEC(SP)                                                                                  \
         if (spt == SP) {                                                                          \
-            if (smem_s > 65536)                                                                   \
-                (void)hipFuncSetAttribute((const void *)&k_elem_spectra<SP>,                      \
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_s); \
-            hipLaunchKernelGGL((k_elem_spectra<SP>), dim3(nb), dim3(kStrainThreads), smem_s, st, db, pc, u0, \
+            using E = ElemFft<256 * SP>;                                                          \
+            /* shares of the traces: about 8,192 workgroups when a launch has few elements */     \
+            const int ng = (J + E::G - 1) / E::G, parts = std::max(1, std::min(ng, 8192 / nb));   \
+            if (E::smem > 65536)                                                                  \
+                (void)hipFuncSetAttribute((const void *)&k_elem_spectra<256 * SP>,                \
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)E::smem); \
+            hipLaunchKernelGGL((k_elem_spectra<256 * SP>), dim3(nb, parts), dim3(E::BLK), E::smem, st, db, pc, u0, \
                                nerun, erun_elem, G.twq_d.p, G.Uspec.p);                           \
             launched = true;                                                                      \
         }
@@ -1197,7 +1199,12 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
         for (auto &e : ev) HIPCHECK(hipEventCreate(&e));
         G.kev.push_back(ev);
         HIPCHECK(hipEventRecord(ev[0], st));
-        SPEC(1) SPEC(2) SPEC(4) SPEC(8) SPEC(16)
+        if (spt == 1) {
+            hipLaunchKernelGGL(k_elem_spectra_short, dim3(nb), dim3(kStrainThreads), 2 * (size_t)pc.M * sizeof(double2),
+                               st, db, pc, u0, nerun, erun_elem, G.twq_d.p, G.Uspec.p);
+            launched = true;
+        }
+        SPEC(2) SPEC(4) SPEC(8) SPEC(16)
 #undef SPEC
         if (!launched) return fail(MCK_EINVAL, "no element-spectra kernel for this trace length");
         HIPCHECK(hipGetLastError());

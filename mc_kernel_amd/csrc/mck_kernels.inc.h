@@ -1519,60 +1519,41 @@ __device__ inline double2 cmul_dd(double2 a, double2 b)
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-// lds_fft in double precision: packs the zero-padded real sequence x (length 2M) as
-// z[n] = x[2n] + i x[2n+1] and runs the length-M Stockham radix-4 FFT (one fused radix-2
-// pass first when log2 M is odd); twiddles from the table in global memory.  Returns the
-// buffer holding Z; ends with a barrier.
-template <int SPT>
-__device__ inline const double2 *lds_fft_d(const double (&x)[SPT], int t0, int nt, int M_, double2 *bufA,
-                                           double2 *bufB, const double2 *__restrict__ twd)
+// lds_fft in double precision for traces of at most 256 samples (one per thread, M = 2 ..
+// 256): packs the zero-padded real sequence x (length 2M) as z[n] = x[2n] + i x[2n+1] and
+// runs the length-M Stockham radix-4 FFT (one fused radix-2 pass first when log2 M is
+// odd); twiddles from the table in global memory.  Returns the buffer holding Z; ends
+// with a barrier.
+__device__ inline const double2 *lds_fft_d(double x, int t0, int nt, int M, double2 *bufA, double2 *bufB,
+                                           const double2 *__restrict__ twd)
 {
-    constexpr int MC = fft_size_of_spt<SPT>();
-    const int M = MC ? MC : M_;
     const int tid = threadIdx.x;
     const int lM = 31 - __clz(M);
     double2 *in = bufA, *ob = bufB;
     int Ns = 1;
     if (lM & 1) {
-        if (SPT >= 2) {
-#pragma unroll
-            for (int q = 0; q < SPT; q += 2) {
-                const int n = (t0 + q) >> 1;
-                if (n < (M >> 1)) {
-                    const double2 z = make_double2(t0 + q < nt ? x[q] : 0.0, t0 + q + 1 < nt ? x[q + 1] : 0.0);
-                    in[2 * n] = z;
-                    in[2 * n + 1] = z;
-                }
-            }
-        } else {
-            double *fa = reinterpret_cast<double *>(ob);
-            for (int n = tid; n < M; n += kStrainThreads) ob[n] = make_double2(0.0, 0.0);
-            __syncthreads();
-            if (t0 < nt) fa[t0] = x[0];
-            __syncthreads();
-            for (int n = tid; n < (M >> 1); n += kStrainThreads) {
-                const double2 z = ob[n];
-                in[2 * n] = z;
-                in[2 * n + 1] = z;
-            }
+        double *fa = reinterpret_cast<double *>(ob);
+        for (int n = tid; n < M; n += kStrainThreads) ob[n] = make_double2(0.0, 0.0);
+        __syncthreads();
+        if (t0 < nt) fa[t0] = x;
+        __syncthreads();
+        for (int n = tid; n < (M >> 1); n += kStrainThreads) {
+            const double2 z = ob[n];
+            in[2 * n] = z;
+            in[2 * n + 1] = z;
         }
         Ns = 2;
     } else {
         for (int n = tid; n < M; n += kStrainThreads) in[n] = make_double2(0.0, 0.0);
         __syncthreads();
         double *fa = reinterpret_cast<double *>(in);
-#pragma unroll
-        for (int q = 0; q < SPT; ++q)
-            if (t0 + q < nt) fa[t0 + q] = x[q];
+        if (t0 < nt) fa[t0] = x;
     }
     __syncthreads();
     const int Mq = M >> 2;
-    // (a compile-time size unrolls the passes and each thread's butterflies)
-    constexpr int UP = MC ? 8 : 1, UJ = MC ? 4 : 1;
-#pragma unroll UP
+#pragma unroll 1
     for (int lNs = Ns == 1 ? 0 : 1; Ns < M; Ns <<= 2, lNs += 2) {
         const int lstride = lM - lNs - 2;            // M / (4 Ns)
-#pragma unroll UJ
         for (int j = tid; j < Mq; j += kStrainThreads) {
             const int kk = j & (Ns - 1);
             const double2 v0 = in[j], v1 = in[j + Mq], v2 = in[j + 2 * Mq], v3 = in[j + 3 * Mq];
@@ -1659,11 +1640,20 @@ __global__ __launch_bounds__(kStrainThreads) void k_strain_traces(
 typedef float vec4f __attribute__((ext_vector_type(4)));
 typedef const float __attribute__((address_space(1))) gfloat;
 typedef const vec4f __attribute__((address_space(1))) gvec4f;
+typedef float vec2f __attribute__((ext_vector_type(2)));
+typedef const vec2f __attribute__((address_space(1))) gvec2f;
 __device__ __forceinline__ float4 gload4(const float *base, int off)
 {
     const vec4f v = *(gvec4f *)((gfloat *)base + (unsigned)off);
     return make_float4(v.x, v.y, v.z, v.w);
 }
+
+__device__ __forceinline__ float2 gload2(const float *base, int off)
+{
+    const vec2f v = *(gvec2f *)((gfloat *)base + (unsigned)off);
+    return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ float gload1(const float *base, int off) { return ((gfloat *)base)[(unsigned)off]; }
 
 // One element pass of k_fwd_traces over all super-tiles: A operands from registers (wa,
 // KS <= 32) or from LDS (sWa[s][64]); WHOLE: nt a multiple of 64 (no partial tile).  The

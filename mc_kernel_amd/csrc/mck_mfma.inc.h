@@ -82,47 +82,287 @@ __global__ void k_group_table(int n, const int *gflag, const int *gpos, const in
 }
 
 // ------------------------------------------------------------------------------------
-// k_elem_spectra: one workgroup per element run u0 + blockIdx.x; the tapered real
-// spectra (x dt) of the element's J = nvar_bwd x 25 nodal traces, U[u - u0][j][k],
-// k <= M, rows ustride apart (zero beyond M).  Computed in double precision and rounded
-// once: the spectra of an element serve all of its pairs.
+// k_elem_spectra: the tapered real spectra (x dt) of the J = nvar_bwd x 25 nodal traces of
+// the elements of runs u0 .. u0 + gridDim.x - 1, U[u - u0][j][k], k <= M, rows ustride
+// apart (zero beyond M).  Computed in double precision and rounded once: the spectra of
+// an element serve all of its pairs.
+//
+// A trace's FFT (z[n] = x[2n] + i x[2n + 1], length M = 512 .. 4096, its upper half zero)
+// runs on M / 16 threads with 16 values each in registers: radix 16, 16 and M / 256
+// (Stockham order), so that it crosses LDS twice instead of once per radix-4 pass, with
+// twiddles kept in registers from trace to trace; the real spectrum's bins k and M - k
+// come from one pair of values.  A workgroup holds G traces at a time; blockIdx.y: a share
+// of the traces, so that few elements still fill the chip.
+// Bound: HBM (25 KB per trace of 2048 samples) and LDS about equally.  3,186 elements of
+// nt 2048 (3.9 GB): 2.73 ms with radix-4 passes through two LDS buffers and twiddles from
+// memory, 1.25 ms (3.1 TB/s; a large copy reaches 4.9); 895 elements of nt 4096 2.76 ->
+// 0.78 ms; 15 elements of nt 1024 184 -> 22 us (their traces spread over workgroups).
 // ------------------------------------------------------------------------------------
-template <int SPT>
-__global__ __launch_bounds__(kStrainThreads) void k_elem_spectra(DevDb db, PathConf pc, int u0, int nrun,
-                                                                 const int *run_elem, const double2 *twd,
-                                                                 float2 *U)
+template <int M>
+struct ElemFft {
+    static constexpr int T = M / 16;                       // threads of a trace
+    static constexpr int BLK = T < 64 ? 64 : T;            // threads of a workgroup
+    static constexpr int G = BLK / T;                      // traces at a time
+    static constexpr int LDS = M + M / 16 + 1;             // padded values of a trace, and z[0] once more
+    static constexpr int R = M / 256;                      // last radix
+    static constexpr size_t smem = (size_t)G * LDS * sizeof(double2);
+};
+
+// LDS slot of value i: one padding slot after every 16 (T is a multiple of 16: slots of
+// i + T q are a constant apart)
+__device__ __forceinline__ int elem_slot(int i) { return i + (i >> 4); }
+__device__ __forceinline__ double2 dadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 dsub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+
+// a (cos, sin) constant: a e^{-i phi}
+__device__ __forceinline__ double2 drot(double2 a, double c, double s)
 {
+#pragma clang fp contract(fast)
+    return make_double2(a.x * c + a.y * s, a.y * c - a.x * s);
+}
+__device__ __forceinline__ double2 dmul(double2 a, double2 b)
+{
+#pragma clang fp contract(fast)
+    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+
+// 4-point DFT (e^{-2 pi i / 4}); HALF: c and d are zero
+template <bool HALF>
+__device__ __forceinline__ void dft4(double2 &a, double2 &b, double2 &c, double2 &d)
+{
+    const double2 s0 = HALF ? a : dadd(a, c), d0 = HALF ? a : dsub(a, c);
+    const double2 s1 = HALF ? b : dadd(b, d), d1 = HALF ? b : dsub(b, d);
+    a = dadd(s0, s1);
+    b = make_double2(d0.x + d1.y, d0.y - d1.x);
+    c = dsub(s0, s1);
+    d = make_double2(d0.x - d1.y, d0.y + d1.x);
+}
+
+// R-point DFT of v[0..R) in place; output r is v[dft_at<R>(r)].  HALF: the upper half of
+// the inputs is zero (R 16)
+template <int R>
+__host__ __device__ constexpr int dft_at(int r) { return R == 16 ? (r >> 2) + 4 * (r & 3) : (R == 8 ? (r >> 2) + 2 * (r & 3) : r); }
+
+template <int R, bool HALF = false>
+__device__ __forceinline__ void dft(double2 *v)
+{
+    constexpr double c8 = 0.70710678118654752440, c16 = 0.92387953251128675613, s16 = 0.38268343236508977173;
+    if constexpr (R == 2) {
+        const double2 a = v[0], b = v[1];
+        v[0] = dadd(a, b);
+        v[1] = dsub(a, b);
+    } else if constexpr (R == 4) {
+        dft4<false>(v[0], v[1], v[2], v[3]);
+    } else if constexpr (R == 8) {
+        dft4<false>(v[0], v[2], v[4], v[6]);
+        dft4<false>(v[1], v[3], v[5], v[7]);
+        v[3] = drot(v[3], c8, c8);
+        v[5] = make_double2(v[5].y, -v[5].x);
+        v[7] = drot(v[7], -c8, c8);
+#pragma unroll
+        for (int r = 0; r < 8; r += 2) {
+            const double2 a = v[r], b = v[r + 1];
+            v[r] = dadd(a, b);
+            v[r + 1] = dsub(a, b);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) dft4<HALF>(v[q], v[q + 4], v[q + 8], v[q + 12]);
+        v[5] = drot(v[5], c16, s16);
+        v[6] = drot(v[6], c8, c8);
+        v[7] = drot(v[7], s16, c16);
+        v[9] = drot(v[9], c8, c8);
+        v[10] = make_double2(v[10].y, -v[10].x);
+        v[11] = drot(v[11], -c8, c8);
+        v[13] = drot(v[13], s16, c16);
+        v[14] = drot(v[14], -c8, c8);
+        v[15] = drot(v[15], -c16, -s16);
+#pragma unroll
+        for (int q = 0; q < 16; q += 4) dft4<false>(v[q], v[q + 1], v[q + 2], v[q + 3]);
+    }
+}
+
+// v[q] *= w^q, q = 1 .. R - 1, from w^1, w^2, w^4, w^8
+template <int R>
+__device__ __forceinline__ void elem_twiddle(double2 *v, const double2 *w)
+{
+    v[1] = dmul(v[1], w[0]);
+    if constexpr (R >= 4) {
+        const double2 w3 = dmul(w[0], w[1]);
+        v[2] = dmul(v[2], w[1]);
+        v[3] = dmul(v[3], w3);
+        if constexpr (R >= 8) {
+            const double2 w5 = dmul(w[0], w[2]), w6 = dmul(w[1], w[2]), w7 = dmul(w3, w[2]);
+            v[4] = dmul(v[4], w[2]);
+            v[5] = dmul(v[5], w5);
+            v[6] = dmul(v[6], w6);
+            v[7] = dmul(v[7], w7);
+            if constexpr (R >= 16) {
+                v[8] = dmul(v[8], w[3]);
+                v[9] = dmul(v[9], dmul(w[0], w[3]));
+                v[10] = dmul(v[10], dmul(w[1], w[3]));
+                v[11] = dmul(v[11], dmul(w3, w[3]));
+                v[12] = dmul(v[12], dmul(w[2], w[3]));
+                v[13] = dmul(v[13], dmul(w5, w[3]));
+                v[14] = dmul(v[14], dmul(w6, w[3]));
+                v[15] = dmul(v[15], dmul(w7, w[3]));
+            }
+        }
+    }
+}
+
+template <int M>
+__global__ __launch_bounds__(ElemFft<M>::BLK, 2) void k_elem_spectra(DevDb db, PathConf pc, int u0, int nrun,
+                                                                     const int *run_elem,
+                                                                     const double2 *__restrict__ twd, float2 *U)
+{
+    using E = ElemFft<M>;
+    constexpr int T = E::T, R = E::R, NB = 16 / R, N = 2 * M, lq = 30 - __builtin_clz(M);    // 2^lq = N / 4
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    double2 *bufA = reinterpret_cast<double2 *>(smem_raw);
-    double2 *bufB = bufA + pc.M;
     const int u = u0 + (int)blockIdx.x;
     if (u >= nrun) return;
-    const int e = run_elem[u];
-    const float *ue = elem_u(db, e);
+    const float *ue = elem_u(db, run_elem[u]);
     if (!ue) return;
-    const int tid = threadIdx.x, nt = pc.nt, t0 = tid * SPT;
-    const int M = fft_size_of_spt<SPT>() ? fft_size_of_spt<SPT>() : pc.M;      // (= pc.M)
+    const int g = (int)threadIdx.x / T, t = (int)threadIdx.x % T;
+    double2 *z = reinterpret_cast<double2 *>(smem_raw) + g * E::LDS;
+    const int J = pc.nvar_bwd * 25, nt = pc.nt;
+    const bool pairs = (nt & 1) == 0;                      // sample pairs aligned
+    // twiddle powers 1, 2, 4, 8 of the second pass (w_256^(t % 16)) and of the NB last
+    // butterflies (w_M^j, j = t + T b)
+    double2 wb[4], wc[NB][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        wb[i] = twiddle_d(twd, ((t & 15) << i) * (N / 256), lq);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+            if ((1 << i) < R) wc[b][i] = twiddle_d(twd, ((t + T * b) << i) * 2, lq);
+    }
+    float2 *Uu = U + (size_t)(u - u0) * J * pc.ustride;
+    // this block's share of the traces, G at a time
+    const int ng = (J + E::G - 1) / E::G;
+    const int i0 = (int)blockIdx.y * ng / (int)gridDim.y, i1 = ((int)blockIdx.y + 1) * ng / (int)gridDim.y;
+    float nx[16];
+    auto load = [&](int i) {
+        const int j = min(i * E::G + g, J - 1);
+        const int src = (pc.bwd_vars[j / 25] * 25 + j % 25) * nt;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int n = 2 * (t + T * q);
+            nx[2 * q] = nx[2 * q + 1] = 0.0f;
+            if (pairs) {
+                if (n < nt) {
+                    const float2 v = gload2(ue, src + n);
+                    nx[2 * q] = v.x;
+                    nx[2 * q + 1] = v.y;
+                }
+            } else {
+                if (n < nt) nx[2 * q] = gload1(ue, src + n);
+                if (n + 1 < nt) nx[2 * q + 1] = gload1(ue, src + n + 1);
+            }
+        }
+    };
+    if (i0 < i1) load(i0);
+    for (int i = i0; i < i1; ++i) {
+        double2 v[16];
+        // (the products of the twiddle powers and the last pass's twiddles are formed or loaded
+        // for every trace: kept across the loop they would not fit the registers)
+        int k0 = t;
+        asm volatile("" : "+v"(k0), "+v"(wb[0].x), "+v"(wb[1].x), "+v"(wb[2].x), "+v"(wb[3].x));
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+                if ((1 << p) < R) asm volatile("" : "+v"(wc[b][p].x));
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            v[q] = make_double2((double)nx[2 * q], (double)nx[2 * q + 1]);
+            const int n = 2 * (t + T * q);
+            if (n < pc.ntaper || n + 1 >= nt - pc.ntaper) {
+                float tp[2];
+                taper_factors(n, nt, pc, tp);
+                v[q].x *= tp[0];
+                v[q].y *= tp[1];
+            }
+            v[q + 8] = make_double2(0.0, 0.0);
+        }
+        if (i + 1 < i1) load(i + 1);
+        dft<16, true>(v);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[17 * t + r] = v[dft_at<16>(r)];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = z[elem_slot(t) + q * (T + T / 16)];
+        __syncthreads();
+        elem_twiddle<16>(v, wb);
+        dft<16>(v);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[(t >> 4) * 272 + (t & 15) + 17 * r] = v[dft_at<16>(r)];
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int q = 0; q < R; ++q) v[b * R + q] = z[elem_slot(t) + b * (T + T / 16) + 272 * q];
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            elem_twiddle<R>(v + b * R, wc[b]);
+            dft<R>(v + b * R);
+#pragma unroll
+            for (int r = 0; r < R; ++r) z[elem_slot(t) + b * (T + T / 16) + 272 * r] = v[b * R + dft_at<R>(r)];
+        }
+        if (t == 0) z[E::LDS - 1] = v[dft_at<R>(0)];
+        __syncthreads();
+        // X_k = E_k + w_N^k O_k and X_(M - k) = conj(E_k - w_N^k O_k)
+        const int j = i * E::G + g;
+        if (j < J) {
+            float2 *dst = Uu + (size_t)j * pc.ustride;
+            const double dt = pc.dt;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+#pragma clang fp contract(fast)
+                const int k = t + T * q;
+                const double2 zk = z[elem_slot(t) + q * (T + T / 16)], zm = z[elem_slot(M - t) - q * (T + T / 16)];
+                const double2 w = twd[k0 + T * q];
+                const double ex = 0.5 * (zk.x + zm.x), ey = 0.5 * (zk.y - zm.y);
+                const double ox = 0.5 * (zk.y + zm.y), oy = 0.5 * (zm.x - zk.x);
+                const double px = w.x * ox - w.y * oy, py = w.x * oy + w.y * ox;
+                dst[k] = make_float2((float)((ex + px) * dt), (float)((ey + py) * dt));
+                dst[M - k] = make_float2((float)((ex - px) * dt), (float)((py - ey) * dt));
+            }
+            if (t == 0) {
+                const double2 zh = z[elem_slot(M / 2)];
+                dst[M / 2] = make_float2((float)(zh.x * dt), (float)(-zh.y * dt));
+            }
+            for (int k = M + 1 + t; k < pc.ustride; k += T) dst[k] = make_float2(0.0f, 0.0f);
+        }
+        __syncthreads();
+    }
+}
+
+// the same for traces of at most 256 samples (M = 2 .. 256): one workgroup per element run,
+// one sample per thread
+__global__ __launch_bounds__(kStrainThreads) void k_elem_spectra_short(DevDb db, PathConf pc, int u0, int nrun,
+                                                                       const int *run_elem, const double2 *twd,
+                                                                       float2 *U)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int M = pc.M;
+    double2 *bufA = reinterpret_cast<double2 *>(smem_raw);
+    double2 *bufB = bufA + M;
+    const int u = u0 + (int)blockIdx.x;
+    if (u >= nrun) return;
+    const float *ue = elem_u(db, run_elem[u]);
+    if (!ue) return;
+    const int tid = threadIdx.x, nt = pc.nt;
     const size_t blk = (size_t)25 * nt;
-    float tap[SPT];
-    taper_factors(t0, nt, pc, tap);
+    float tap[1];
+    taper_factors(tid, nt, pc, tap);
     const int J = pc.nvar_bwd * 25;
-    const bool full_vec = (t0 + SPT <= nt) && ((nt & 3) == 0) && (SPT % 4) == 0;
     float2 *Uu = U + (size_t)(u - u0) * J * pc.ustride;
     for (int j = 0; j < J; ++j) {
-        const float *src = ue + (size_t)pc.bwd_vars[j / 25] * blk + (size_t)(j % 25) * nt + t0;
-        double x[SPT];
-        if (full_vec) {
-#pragma unroll
-            for (int q = 0; q < SPT; q += 4) {
-                const float4 v = *reinterpret_cast<const float4 *>(src + q);
-                x[q] = (double)v.x * tap[q]; x[q + 1] = (double)v.y * tap[q + 1];
-                x[q + 2] = (double)v.z * tap[q + 2]; x[q + 3] = (double)v.w * tap[q + 3];
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < SPT; ++q) x[q] = (t0 + q < nt) ? (double)src[q] * tap[q] : 0.0;
-        }
-        const double2 *Z = lds_fft_d(x, t0, nt, M, bufA, bufB, twd);
+        const float *src = ue + (size_t)pc.bwd_vars[j / 25] * blk + (size_t)(j % 25) * nt;
+        const double x = tid < nt ? (double)src[tid] * tap[0] : 0.0;
+        const double2 *Z = lds_fft_d(x, tid, nt, M, bufA, bufB, twd);
         float2 *dst = Uu + (size_t)j * pc.ustride;
         for (int k = tid; k < pc.ustride; k += kStrainThreads)
             dst[k] = k <= M ? rfft_bin_d(Z, k, M, twd, pc.dt) : make_float2(0.0f, 0.0f);
