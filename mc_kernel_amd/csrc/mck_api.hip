@@ -870,12 +870,12 @@ int build_kernels(State &G) {
                         rd.cls_pos[q] = n;
                         rd.cls_h[n++] = rd.slot_h[q];
                     }
-                while ((n - b) & 15) { rd.cls_h[n] = rd.cls_h[b]; ++n; }
+                while ((n - b) & 3) { rd.cls_h[n] = rd.cls_h[b]; ++n; }
                 rd.cls_end[c] = n;
             }
         }
         pc.max_slots = 1;
-        pc.max_cls = 16;
+        pc.max_cls = 4;
         for (int r = 0; r < G.R; ++r) {
             pc.max_slots = std::max(pc.max_slots, lr[r].nslot);
             pc.max_cls = std::max(pc.max_cls, lr[r].cls_end[2]);
@@ -1170,11 +1170,11 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
     if (G.bwd_path_env < 0 && G.cost_pair_us * npairs < G.cost_group_us * ngroups + G.cost_run_us * nerun)
         return launch_status(launch_bwd(G, db, npairs, order, loc_b, Wb, Qb, phys, base_out, active, P));
     G.stats.mfma_runs += nerun;
-    const int J = pc.nvar_bwd * 25, KS = mfma_ks(J);
+    const int J = pc.nvar_bwd * 25, KS = mfma_ks(pc.nvar_bwd), NBLK = mfma_nblock(pc.nd_b, pc.nvar_bwd);
     const size_t per_elem = (size_t)J * pc.ustride * sizeof(float2);
     const int batch = (int)std::max<size_t>(1, std::min<size_t>((size_t)nerun, G.uspec_budget / per_elem));
     HIPCHECK(G.Uspec.ensure((size_t)batch * J * pc.ustride));
-    const size_t smem_m = mfma_wave_lds(KS, pc.nd_b, pc.max_cls);
+    const size_t smem_m = mfma_group_lds(NBLK, pc.max_cls, kMfmaWaves);
     const int spt = spt_for(pc.nt);
     G.stats.spt = spt;
     G.stats.nd_f = pc.nd_f;
@@ -1212,15 +1212,17 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
         launched = false;
         // W waves per element run sharing its spectra through LDS, or one wave per group
         int W = G.mfma_waves;
-        if (W > 1 && mfma_wg_lds(KS, pc.nd_b, pc.max_cls, W) > 160 * 1024) W = W > 2 ? 2 : 1;
-        if (W > 1 && mfma_wg_lds(KS, pc.nd_b, pc.max_cls, W) > 160 * 1024) W = 1;
-        const size_t smem_w = mfma_wg_lds(KS, pc.nd_b, pc.max_cls, W);
-#define EVAL1(NF, NB, NV)                                                                         \
-        if (pc.nd_f == NF && pc.nd_b == NB && pc.nvar_bwd == NV) {                                \
+        if (W > 1 && mfma_wg_lds(KS, NBLK, pc.max_cls, W) > 160 * 1024) W = W > 2 ? 2 : 1;
+        if (W > 1 && mfma_wg_lds(KS, NBLK, pc.max_cls, W) > 160 * 1024) W = 1;
+        const size_t smem_w = mfma_wg_lds(KS, NBLK, pc.max_cls, W);
+        // slot groups in registers: those of the largest receiver, up to 8
+        const int ng = std::min(kMfmaMaxRegGroups, 2 * ((pc.max_cls / 4 + 1) / 2));
+#define EVAL1(NF, NB, NV, NG)                                                                     \
+        if (ng == NG && pc.nd_f == NF && pc.nd_b == NB && pc.nvar_bwd == NV) {                                \
             if (smem_m > 65536)                                                                   \
-                (void)hipFuncSetAttribute((const void *)&k_bwd_mfma<NF, NB, NV>,                  \
+                (void)hipFuncSetAttribute((const void *)&k_bwd_mfma<NF, NB, NV, NG>,                  \
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_m); \
-            hipLaunchKernelGGL((k_bwd_mfma<NF, NB, NV>), dim3(grid_x8(ngroups)), dim3(64), smem_m, st, pc, u0, nb, \
+            hipLaunchKernelGGL((k_bwd_mfma<NF, NB, NV, NG>), dim3(grid_x8(ngroups)), dim3(64 * kMfmaWaves), smem_m, st, pc, u0, nb, \
                                ngroups, group_first, group_erun, G.Uspec.p, order, R, Wb, Qb, G.opQf.p, \
                                G.Fspec.p, recs, kerns, G.Hp.p, pc.max_cls, G.model_idx.p, G.model.p, \
                                G.S.model_ndepth, G.S.relative_kernel, G.nk, phys, base_out, G.xyz.p, \
@@ -1240,7 +1242,8 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
             launched = true;                                                                      \
         }
 #define EVAL(NF, NB, NV) \
-        if (W == 1) { EVAL1(NF, NB, NV) } else { EVALW(NF, NB, NV, 2) EVALW(NF, NB, NV, 4) }
+        if (W == 1) { EVAL1(NF, NB, NV, 2) EVAL1(NF, NB, NV, 4) EVAL1(NF, NB, NV, 6) EVAL1(NF, NB, NV, 8) }       \
+        else { EVALW(NF, NB, NV, 2) EVALW(NF, NB, NV, 4) }
         EVAL(1, 1, 2) EVAL(1, 1, 3) EVAL(4, 4, 2) EVAL(6, 4, 2) EVAL(4, 6, 3) EVAL(6, 6, 3)
 #undef EVAL
 #undef EVALW

@@ -73,8 +73,8 @@ struct Located {
 // Path-wide configuration passed by value to the kernels.
 struct PathConf {
     int nt, M, nomega;        // samples, FFT half length (N/2) and N/2+1
-    int ustride;              // row stride of element spectra: nomega rounded up to 16
-    int fstride;              // row stride of forward and window spectra (= ustride)
+    int ustride;              // bins of an element spectrum: nomega rounded up to 16
+    int fstride;              // bins of a forward and a window spectrum (= ustride)
     double dt;
     int nd;                   // 1 (trace) or 6 (full strain)
     int full;
@@ -108,6 +108,11 @@ struct PathConf {
     double damp_radius;
     double src_r[3];
 };
+
+// Forward and element spectra are stored by tiles of 16 bins, the n components (traces) of a
+// tile together, so that what a tile of the contraction reads is contiguous: the offset
+// of bin k of component c
+__host__ __device__ constexpr size_t tile_at(int n, int c, int k) { return ((size_t)(k >> 4) * n + c) * 16 + (k & 15); }
 
 // LDS layout of the per-point operator set-up
 struct OpShared {
@@ -152,10 +157,10 @@ struct RecDesc {
     int grp_h[kMaxSlots], grp_first[kMaxSlots], grp_n[kMaxSlots];
     // the slots by base-kernel class for the matrix-core kernel: lambda (slot_bk 0), mu
     // (1), combinations; class c holds the positions c ? cls_end[c - 1] : 0 .. cls_end[c] - 1,
-    // each class padded to a multiple of 16 positions (blocks of 16 matrix-core columns;
+    // each class padded to a multiple of 4 positions (groups of 4 matrix-core columns;
     // padding: another position's window spectrum, a sum nobody reads); cls_h: window
     // spectrum of a position, cls_pos: position of a slot
-    int cls_h[kMaxSlots + 48];
+    int cls_h[kMaxSlots + 12];
     int cls_pos[kMaxSlots];
     int cls_end[3];
 };

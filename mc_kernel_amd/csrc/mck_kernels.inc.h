@@ -1788,7 +1788,8 @@ __global__ __launch_bounds__(64, 2) void k_fwd_traces(DevDb db, PathConf pc, int
 // The point's strain traces (k_fwd_traces: T[sorted item][ND][nt]), cumsum
 // (simple_routines.f90:314-341), taper + zero pad (fft.f90:546-601) and LDS real FFT
 // (fft.f90:375-413).
-// F: [point][ND][fstride] spectra of the carried source-frame components (bins < nomega).
+// F: [point][fstride / 16][ND][16] spectra of the carried source-frame components (tile_at;
+// zero past nomega).
 // ------------------------------------------------------------------------------------
 template <int SPT, int ND>
 __global__ __launch_bounds__(kStrainThreads, (SPT <= 8 && ND <= 4) ? 3 : (SPT <= 8 ? 2 : 1)) void k_fwd_spectra(
@@ -1846,9 +1847,9 @@ __global__ __launch_bounds__(kStrainThreads, (SPT <= 8 && ND <= 4) ? 3 : (SPT <=
 #pragma unroll
         for (int q = 0; q < SPT; ++q) x[q] *= tap[q];
         const float2 *Z = lds_fft(x, t0, nt, M, bufA, bufB, Tq);
-        float2 *dst = F + ((size_t)p * ND + c) * pc.fstride;
+        float2 *dst = F + (size_t)p * ND * pc.fstride;
         for (int k = tid; k < pc.fstride; k += kStrainThreads)
-            dst[k] = k <= M ? rfft_bin(Z, k, M, Tq, fdt) : make_float2(0.0f, 0.0f);
+            dst[tile_at(ND, c, k)] = k <= M ? rfft_bin(Z, k, M, Tq, fdt) : make_float2(0.0f, 0.0f);
         __syncthreads();
     }
 }
@@ -1965,7 +1966,7 @@ __global__ __launch_bounds__(kStrainThreads, (SPT <= 8 && NDB <= 4) ? 3 : (SPT <
             const bool ok = j < SPT ? (k < M) : (j == SPT && tid == kM_owner);
 #pragma unroll
             for (int c = 0; c < NDF; ++c)
-                fv[jj][c] = (j < NJ && ok) ? Fp[(size_t)c * pc.fstride + k] : make_float2(0.f, 0.f);
+                fv[jj][c] = (j < NJ && ok) ? Fp[tile_at(NDF, c, k)] : make_float2(0.f, 0.f);
         }
 #pragma unroll
         for (int jj = 0; jj < JB; ++jj) {

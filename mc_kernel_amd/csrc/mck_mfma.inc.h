@@ -10,7 +10,7 @@
 // The nodal spectra U of every backward element a launch touches are computed once
 // (k_elem_spectra, one workgroup per element); the pairs of an element then form their
 // spectra as one matrix product [bins x traces] x [traces x pairs] on the matrix cores
-// (fp32 operands as split fp16 products, kMfmaSplit), fused with the frequency-domain contraction of
+// (fp32 operands as split fp16 products), fused with the frequency-domain contraction of
 // k_bwd_eval: base kernels per bin (kernel.f90:514-570) against the forward spectra of
 // the pair's point, the filtered window integrals sum_k Re(bk_k H_k) accumulated in FP64
 // (kernel.f90:410-510, 946-1020), and the physical kernels (kernel.f90:665-832).
@@ -23,7 +23,7 @@ namespace mck {
 
 // Work tables of element- and receiver-sorted pair keys (element * R + receiver):
 // element runs (the elements whose spectra a launch needs) and groups of at most 16
-// consecutive pairs with one key (one wave of k_bwd_mfma each).
+// consecutive pairs with one key (one workgroup of k_bwd_mfma each).
 // flags: eflag[i] = a new element starts at i, kflag[i] = a new key starts at i
 __global__ void k_run_flags(int n, const int *keys, int R, int *eflag, int *kflag)
 {
@@ -83,9 +83,9 @@ __global__ void k_group_table(int n, const int *gflag, const int *gpos, const in
 
 // ------------------------------------------------------------------------------------
 // k_elem_spectra: the tapered real spectra (x dt) of the J = nvar_bwd x 25 nodal traces of
-// the elements of runs u0 .. u0 + gridDim.x - 1, U[u - u0][j][k], k <= M, rows ustride
-// apart (zero beyond M).  Computed in double precision and rounded once: the spectra of
-// an element serve all of its pairs.
+// the elements of runs u0 .. u0 + gridDim.x - 1, U[u - u0][tile][j][16 bins] (tile_at; zero
+// beyond bin M).  Computed in double precision and rounded once: the spectra of an
+// element serve all of its pairs.
 //
 // A trace's FFT (z[n] = x[2n] + i x[2n + 1], length M = 512 .. 4096, its upper half zero)
 // runs on M / 16 threads with 16 values each in registers: radix 16, 16 and M / 256
@@ -315,25 +315,25 @@ __global__ __launch_bounds__(ElemFft<M>::BLK, 2) void k_elem_spectra(DevDb db, P
         // X_k = E_k + w_N^k O_k and X_(M - k) = conj(E_k - w_N^k O_k)
         const int j = i * E::G + g;
         if (j < J) {
-            float2 *dst = Uu + (size_t)j * pc.ustride;
+            // (T is a multiple of 16: the bins t + T q and M - t - T q are T J apart)
+            float2 *dk = Uu + tile_at(J, j, t), *dm = Uu + tile_at(J, j, M - t);
             const double dt = pc.dt;
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
 #pragma clang fp contract(fast)
-                const int k = t + T * q;
                 const double2 zk = z[elem_slot(t) + q * (T + T / 16)], zm = z[elem_slot(M - t) - q * (T + T / 16)];
                 const double2 w = twd[k0 + T * q];
                 const double ex = 0.5 * (zk.x + zm.x), ey = 0.5 * (zk.y - zm.y);
                 const double ox = 0.5 * (zk.y + zm.y), oy = 0.5 * (zm.x - zk.x);
                 const double px = w.x * ox - w.y * oy, py = w.x * oy + w.y * ox;
-                dst[k] = make_float2((float)((ex + px) * dt), (float)((ey + py) * dt));
-                dst[M - k] = make_float2((float)((ex - px) * dt), (float)((py - ey) * dt));
+                dk[(size_t)q * T * J] = make_float2((float)((ex + px) * dt), (float)((ey + py) * dt));
+                dm[-(ptrdiff_t)q * T * J] = make_float2((float)((ex - px) * dt), (float)((py - ey) * dt));
             }
             if (t == 0) {
                 const double2 zh = z[elem_slot(M / 2)];
-                dst[M / 2] = make_float2((float)(zh.x * dt), (float)(-zh.y * dt));
+                Uu[tile_at(J, j, M / 2)] = make_float2((float)(zh.x * dt), (float)(-zh.y * dt));
             }
-            for (int k = M + 1 + t; k < pc.ustride; k += T) dst[k] = make_float2(0.0f, 0.0f);
+            for (int k = M + 1 + t; k < pc.ustride; k += T) Uu[tile_at(J, j, k)] = make_float2(0.0f, 0.0f);
         }
         __syncthreads();
     }
@@ -363,145 +363,171 @@ __global__ __launch_bounds__(kStrainThreads) void k_elem_spectra_short(DevDb db,
         const float *src = ue + (size_t)pc.bwd_vars[j / 25] * blk + (size_t)(j % 25) * nt;
         const double x = tid < nt ? (double)src[tid] * tap[0] : 0.0;
         const double2 *Z = lds_fft_d(x, tid, nt, M, bufA, bufB, twd);
-        float2 *dst = Uu + (size_t)j * pc.ustride;
         for (int k = tid; k < pc.ustride; k += kStrainThreads)
-            dst[k] = k <= M ? rfft_bin_d(Z, k, M, twd, pc.dt) : make_float2(0.0f, 0.0f);
+            Uu[tile_at(J, j, k)] = k <= M ? rfft_bin_d(Z, k, M, twd, pc.dt) : make_float2(0.0f, 0.0f);
         __syncthreads();
     }
 }
 
 constexpr int kMfmaPairs = 16;         // pairs of one wave (the matrix-core columns)
+constexpr int kMfmaWaves = 4;          // waves of a workgroup of k_bwd_mfma (one group)
 
 // The contraction U W of the element spectra with the pair weights on the fp16 matrix
-// cores (v_mfma_f32_16x16x32_f16, 16 times the fp32 products' rate): every fp32 operand x
-// is split into x_hi = fp16(x) and x_lo = fp16(x - x_hi), 22 of its 24 significant bits,
-// and U W = U_hi W_hi + U_hi W_lo + U_lo W_hi (fp16 products are exact in fp32; the
-// dropped U_lo W_lo is below 2^-22 of a product).  The operands are scaled by powers of
-// two into fp16's range first (W per pair, U per tile of 16 bins, to below 2^14) and the
-// sums scaled back.  K: the traces in blocks of 32 (8 per lane).  false: the fp32
-// products (v_mfma_f32_16x16x4f32, K in steps of 4).
-constexpr bool kMfmaSplit = true;
+// cores (v_mfma_f32_16x16x32_f16): every fp32 operand x is split into x_hi = fp16(x) and
+// x_lo = fp16(x - x_hi), 22 of its 24 significant bits, and U W = U_hi W_hi + U_hi W_lo +
+// U_lo W_hi (fp16 products are exact in fp32; the dropped U_lo W_lo is below 2^-22 of a
+// product).  The operands are scaled by powers of two into fp16's range first (W per pair,
+// U per tile of 16 bins, to below 2^14) and the base kernels scaled back.  K: one block of
+// 32 per variable, its 25 nodal traces (8 per lane) and 7 zeros, so that a component skips
+// the variables its strain does not contain.
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-// A operands per lane for J traces (trace mfma_trace(s, g) in slot s of lane group g)
-__host__ __device__ constexpr int mfma_ks(int J) { return kMfmaSplit ? 8 * ((J + 31) / 32) : (J + 3) / 4; }
-__device__ __forceinline__ int mfma_trace(int s, int g)
+constexpr int mfma_ks(int nvb) { return 8 * nvb; }     // element spectra per lane
+
+// whether carried component c contains variable v (sem_derivatives.f90:281-649): monopole
+// fields (u_s, u_z: ss, pp, zz, sz), dipole fields (u_s, u_p, u_z: the Voigt six), traces
+__host__ __device__ constexpr bool mfma_has(int ndb, int v, int c)
 {
-    return kMfmaSplit ? 32 * (s >> 3) + 8 * g + (s & 7) : 4 * s + g;
+    if (ndb == 1) return true;
+    if (ndb == 4) return v == 0 ? c != 2 : c >= 2;
+    return v == 0 ? (c != 2 && c != 3) : (v == 1 ? (c == 1 || c == 3 || c == 5) : (c >= 2 && c <= 4));
 }
+// index of (v, c) among the blocks a group's weights are stored in, and their number
+__host__ __device__ constexpr int mfma_wblock(int ndb, int v, int c)
+{
+    int n = 0;
+    for (int i = 0; i < v * ndb + c; ++i) n += mfma_has(ndb, i / ndb, i % ndb) ? 1 : 0;
+    return n;
+}
+__host__ __device__ constexpr int mfma_nblock(int ndb, int nvb) { return mfma_wblock(ndb, nvb, 0); }
 
 // the largest of a non-negative value over the wave (all 64 lanes active): within each
 // row of 16 lanes by DPP (lane swaps 1 and 2, rotations by 4 and 8), then across the 4
 // rows on the bit patterns (non-negative floats order as unsigned integers)
 __device__ __forceinline__ float mfma_wave_max(float x)
 {
-    int v = __builtin_bit_cast(int, x);
-    v = __builtin_bit_cast(int, fmaxf(__builtin_bit_cast(float, v),
-                                      __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false))));
-    v = __builtin_bit_cast(int, fmaxf(__builtin_bit_cast(float, v),
-                                      __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false))));
-    v = __builtin_bit_cast(int, fmaxf(__builtin_bit_cast(float, v),
-                                      __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, v, 0x124, 0xF, 0xF, false))));
-    v = __builtin_bit_cast(int, fmaxf(__builtin_bit_cast(float, v),
-                                      __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, false))));
-    const unsigned r0 = (unsigned)__builtin_amdgcn_readlane(v, 0), r1 = (unsigned)__builtin_amdgcn_readlane(v, 16);
-    const unsigned r2 = (unsigned)__builtin_amdgcn_readlane(v, 32), r3 = (unsigned)__builtin_amdgcn_readlane(v, 48);
+    unsigned v = __builtin_bit_cast(unsigned, x), o;
+    o = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);
+    v = v > o ? v : o;
+    o = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);
+    v = v > o ? v : o;
+    o = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xF, 0xF, true);
+    v = v > o ? v : o;
+    o = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);
+    v = v > o ? v : o;
+    const unsigned r0 = (unsigned)__builtin_amdgcn_readlane((int)v, 0), r1 = (unsigned)__builtin_amdgcn_readlane((int)v, 16);
+    const unsigned r2 = (unsigned)__builtin_amdgcn_readlane((int)v, 32), r3 = (unsigned)__builtin_amdgcn_readlane((int)v, 48);
     const unsigned m = r0 > r1 ? r0 : r1, n = r2 > r3 ? r2 : r3;
     return __builtin_bit_cast(float, m > n ? m : n);
 }
 
-// x (scaled into fp16's range) = hi + lo to 22 bits
-__device__ __forceinline__ void mfma_split(float x, _Float16 &hi, _Float16 &lo)
+// max(m, |a|, |b|) in one instruction (fmaxf would quiet NaNs first)
+__device__ __forceinline__ float mfma_max3(float m, float a, float b)
 {
-    hi = (_Float16)x;
-    lo = (_Float16)(x - (float)hi);
+    float r;
+    asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+    return r;
 }
 
-// LDS bytes of one wave's own arrays: the B operands [KS][NDB][64] of its 16 pairs and the
-// FP64 slot sums of its npos class positions (npos / 16 blocks of 16 x 16)
-__host__ __device__ constexpr size_t mfma_wave_lds(int ks, int ndb, int npos)
+// x, y (scaled into fp16's range) = hi + lo to 22 bits, as packed halves: fp16 conversion in
+// pairs and the remainders by one mixed-precision FMA each (exact)
+__device__ __forceinline__ void mfma_split2(float x, float y, unsigned &hi, unsigned &lo)
 {
-    return (size_t)ks * ndb * 64 * sizeof(float) + (size_t)npos * kMfmaPairs * sizeof(double);
+    float rx, ry;
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(hi) : "v"(x), "v"(y));
+    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(rx) : "v"(hi), "v"(x));
+    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(ry) : "v"(hi), "v"(y));
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(lo) : "v"(rx), "v"(ry));
+}
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+// LDS bytes of a group's arrays: the B operands of its 16 pairs (nblock blocks, high and
+// low halves) and the FP64 slot sums of its npos class positions, one set per wave
+__host__ __device__ constexpr size_t mfma_group_lds(int nblock, int npos, int waves)
+{
+    return (size_t)nblock * 2 * 64 * sizeof(v8h) + (size_t)waves * npos * kMfmaPairs * sizeof(double);
 }
 
-// the slot sum of class position pos for pair jp, from the blocks of matrix-core results
-// (block pos / 16: D[pair][pos % 16] in lane pos % 16 + 16 (pair % 4), element pair / 4)
+// the slot sum of class position pos for pair jp, from the groups of matrix-core results
+// (group pos / 4: D[pair][pos % 4] in lane pos % 4 + 4 (pair / 4) + 16 (pair % 4))
 __device__ __forceinline__ double mfma_slot_sum(const double *sAcc, int pos, int jp)
 {
-    return sAcc[(size_t)(pos >> 4) * 256 + 4 * ((pos & 15) + 16 * (jp & 3)) + (jp >> 2)];
+    return sAcc[(pos >> 2) * 64 + (pos & 3) + 4 * (jp >> 2) + 16 * (jp & 3)];
 }
 
 // LDS bytes of k_bwd_mfma_wg with w waves: two 16-bin tiles of the element spectra
 // [4 KS][16] and every wave's own arrays
-__host__ __device__ constexpr size_t mfma_wg_lds(int ks, int ndb, int npos, int w)
+__host__ __device__ constexpr size_t mfma_wg_lds(int ks, int nblock, int npos, int w)
 {
-    return 2 * (size_t)ks * 4 * 16 * sizeof(float2) + (size_t)w * mfma_wave_lds(ks, ndb, npos);
+    return 2 * (size_t)ks * 4 * 16 * sizeof(float2) + (size_t)w * mfma_group_lds(nblock, npos, 1);
 }
 
-// One wave's group: its pairs (lane l holds pair l % 16), their receiver and the
-// per-pair coefficients F.B = f^T Amu b (earth frame through the rotations of the point,
-// Qf, and of the pair, Qb) and the traces uf.f, ub.b
+// One wave's group: its pairs (lane l holds pair l % 16), their receiver and the per-pair
+// coefficients F.B = f^T Amu b (earth frame through the rotations of the point, Qf, and of
+// the pair, Qb); the traces are f0 + f1 + f2 and b0 + b1 + b2 (the diagonal components,
+// invariant under the rotations)
 template <int NDF, int NDB>
 struct MfmaGroup {
     int g0, n, r, p;
-    int ew;                             // the pair's weights scaled by 2^ew (split products)
+    int ew;                             // the pair's weights scaled by 2^ew
     bool valid;
-    float uf[NDF], ub[NDB], Amu[NDF][NDB];
+    float Amu[NDF][NDB];
 };
 
-// Loads group grp: its B operands into sW (fp32 products: sW[(s NDB + c) 64 + l'] = W of
-// pair l' % 16, component c, trace 4 s + l' / 16; split products: the v8h at
-// ((kb NDB + c) 2 + part) 64 + l' holds part hi / lo of 2^ew W of pair l' % 16, component c,
-// traces 32 kb + 8 (l' / 16) + q, q = 0..7; zero past the group or the traces), its slot
-// sums zeroed, its coefficients.  Called by the 64 lanes of the wave; the caller
-// synchronises before sW or sAcc is read.
-template <int NDF, int NDB, int NVB>
+// Loads group grp: its B operands into sW (the v8h at (2 block + part) 64 + l' holds part
+// hi / lo of 2^ew W of pair l' % 16 and the block's component and variable, traces
+// 8 (l' / 16) + q, q = 0..7; zero past the group or the 25 traces), its slot sums zeroed, its
+// coefficients.  Called by the 64 lanes of each of the group's NW waves (wv: which; the
+// waves share sW, each has its own sAcc); the caller synchronises before sW or sAcc is read.
+template <int NDF, int NDB, int NVB, int NW>
 __device__ __forceinline__ void mfma_group_setup(MfmaGroup<NDF, NDB> &G, int grp, const int *group_first,
                                                  const int *order, int R, const float *Wb, const float *Qb,
-                                                 const float *Qf, const PathConf &pc, int npos, float *sW,
-                                                 double *sAcc, int l)
+                                                 const float *Qf, const PathConf &pc, int npos, v8h *sW,
+                                                 double *sAcc, int l, int wv)
 {
-    constexpr int J = NVB * 25, KS = mfma_ks(J);
-    const int jp = l & 15;
+    constexpr int J = NVB * 25;
+    const int jp = l & 15, g = l >> 4;
     G.g0 = group_first[grp];
     G.n = group_first[grp + 1] - G.g0;
-    if constexpr (kMfmaSplit) {
-        // the pair's scale: its largest weight to below 2^14 (lanes jp, jp + 16, .. share it)
-        const float *wp = Wb + (size_t)(G.g0 + jp) * NDB * J;
-        float mx = 0.0f;
-        if (jp < G.n)
-            for (int i = l >> 4; i < NDB * J; i += 4) mx = fmaxf(mx, fabsf(wp[i]));
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        int e;
-        (void)frexpf(mx, &e);
-        G.ew = 14 - e;
-        v8h *sWh = reinterpret_cast<v8h *>(sW);
-        const int g = l >> 4;
-        for (int kc = 0; kc < (KS / 8) * NDB; ++kc) {          // kc = kb NDB + c
-            const int kb = kc / NDB, c = kc - kb * NDB;
-            v8h hi, lo;
+    // all weights loaded at once, without branches (past the traces or the group: a valid
+    // weight, then zero)
+    constexpr int NBLK = mfma_nblock(NDB, NVB);
+    const float *wp = Wb + (size_t)(G.g0 + min(jp, G.n - 1)) * NDB * J;
+    float w[NBLK][8], mx = 0.0f;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int j = 32 * kb + 8 * g + q;
-                const float w = (jp < G.n && j < J) ? ldexpf(wp[c * J + j], G.ew) : 0.0f;
-                _Float16 h, o;
-                mfma_split(w, h, o);
-                hi[q] = h;
-                lo[q] = o;
-            }
-            sWh[(2 * kc) * 64 + l] = hi;
-            sWh[(2 * kc + 1) * 64 + l] = lo;
+    for (int v = 0; v < NVB; ++v)
+#pragma unroll
+        for (int c = 0; c < NDB; ++c) {
+            if (!mfma_has(NDB, v, c)) continue;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) w[mfma_wblock(NDB, v, c)][q] = wp[c * J + 25 * v + min(8 * g + q, 24)];
         }
-    } else {
-        G.ew = 0;
-        for (int idx = l; idx < KS * NDB * 64; idx += 64) {
-            const int s = idx / (NDB * 64), rem = idx - s * (NDB * 64), c = rem >> 6, ll = rem & 63;
-            const int pj = ll & 15, j = 4 * s + (ll >> 4);
-            float w = 0.0f;
-            if (pj < G.n && j < J) w = Wb[(size_t)(G.g0 + pj) * NDB * J + c * J + j];
-            sW[idx] = w;
+    // the pair's scale: its largest weight to below 2^14 (lanes jp, jp + 16, .. share it)
+#pragma unroll
+    for (int b = 0; b < NBLK; ++b)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            if (jp >= G.n || 8 * g + q >= 25) w[b][q] = 0.0f;
+            mx = fmaxf(mx, fabsf(w[b][q]));
         }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    int e;
+    (void)frexpf(mx, &e);
+    G.ew = 14 - e;
+#pragma unroll
+    for (int b = 0; b < NBLK; ++b) {
+        if (NW > 1 && b % NW != wv) continue;
+        v4u hi, lo;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            unsigned h, o;
+            mfma_split2(ldexpf(w[b][2 * q], G.ew), ldexpf(w[b][2 * q + 1], G.ew), h, o);
+            hi[q] = h;
+            lo[q] = o;
+        }
+        sW[(2 * b) * 64 + l] = __builtin_bit_cast(v8h, hi);
+        sW[(2 * b + 1) * 64 + l] = __builtin_bit_cast(v8h, lo);
     }
     for (int s = l; s < npos * kMfmaPairs; s += 64) sAcc[s] = 0.0;
     G.valid = jp < G.n;
@@ -518,10 +544,7 @@ __device__ __forceinline__ void mfma_group_setup(MfmaGroup<NDF, NDB> &G, int grp
             for (int c = 0; c < NDB; ++c) qb[i][c] = G.valid ? Qb[(size_t)(G.g0 + jp) * 36 + i * 6 + c] : 0.0f;
         }
 #pragma unroll
-        for (int m = 0; m < NDF; ++m) {
-            // the trace is invariant under the rotations: exactly 1 for the diagonal
-            // components (ss, pp, zz), 0 for the others
-            G.uf[m] = pc.comps_f[m] < 3 ? 1.0f : 0.0f;
+        for (int m = 0; m < NDF; ++m)
 #pragma unroll
             for (int c = 0; c < NDB; ++c) {
                 float a = 0.0f;
@@ -529,186 +552,202 @@ __device__ __forceinline__ void mfma_group_setup(MfmaGroup<NDF, NDB> &G, int grp
                 for (int i = 0; i < 6; ++i) a += qf[i][m] * qb[i][c];
                 G.Amu[m][c] = a;
             }
-        }
-#pragma unroll
-        for (int c = 0; c < NDB; ++c) G.ub[c] = pc.comps_b[c] < 3 ? 1.0f : 0.0f;
     } else {
-        G.uf[0] = 1.0f; G.ub[0] = 1.0f; G.Amu[0][0] = 1.0f;
+        G.Amu[0][0] = 1.0f;
     }
 }
 
-// The slot sums of one tile on the FP64 matrix cores: for every block of 16 class
-// positions (one class, columns c = 0..15: window spectrum cls_h[16 b + c]),
-// D[pair][c] += sum over the tile's 16 bins of Re(bk H) = bk.x H.x + bk.y (-H.y); the
-// fp32 base kernels and window spectra multiply exactly in FP64 and the products are
-// summed in FP64.  This lane holds bk of pair l % 16 at bins kb .. kb + 3 (the A
-// operands: pair l % 16, k = l / 16) and loads column l % 16's spectra at the same bins
-// (the B operands).  D of block b: sAcc[b 256 + 4 l + r] = D[l / 16 + 4 r][l % 16] (the
-// FP64 product's result layout).
-// blocks of slot sums kept in registers across the tiles (the rest in LDS): 2 where the
-// registers still fit two waves per SIMD (4 or 6 forward components, 2 backward variables)
-template <int NDF, int NVB>
-constexpr int mfma_dreg() { return (NDF >= 4 && NVB == 2) ? 2 : 0; }
+// A wave's window spectra and slot sums: per group of 4 class positions (one class), lane l
+// reads column l % 4's spectrum at the bins of its pair (hoff: bytes to the row and the
+// lane's bins) and holds D[pair][column] (mfma_slot_sum's layout).  The first NG groups'
+// sums stay in registers across the tiles (NG: 2, 4, 6 or 8, at least the receivers' groups up
+// to 8; groups past a receiver's are summed into values nobody reads), further ones in LDS.
+// The x and y products have a sum each: two chains of dependent products.
+constexpr int kMfmaMaxRegGroups = 8;
 
-// block b of the tile's slot sums: d + the block's products
-__device__ __forceinline__ v4d mfma_window_block(const float2 (&bk0)[4], const float2 (&bk1)[4], int b, int l,
-                                                 int kb, int fs, const RecDesc &rd, const float2 *Hp, v4d d)
+template <int NG>
+struct MfmaSlots {
+    int ng, e0, e1;                       // groups; end of the lambda and of the mu class
+    unsigned hoff[NG];
+    double accx[NG], accy[NG];
+};
+
+template <int NG>
+__device__ __forceinline__ void mfma_slots_init(MfmaSlots<NG> &S, const RecDesc &rd, int l, int fs)
 {
-    const int p0 = b << 4;
-    const int cls = p0 < rd.cls_end[0] ? 0 : (p0 < rd.cls_end[1] ? 1 : 2);
-    const float4 *src = reinterpret_cast<const float4 *>(Hp + (size_t)rd.cls_h[p0 + (l & 15)] * fs + kb);
-    const float4 q0 = src[0], q1 = src[1];
-    const double2 h[4] = {make_double2(q0.x, q0.y), make_double2(q0.z, q0.w), make_double2(q1.x, q1.y),
-                          make_double2(q1.z, q1.w)};
-    double ax[4], ay[4];
+    S.ng = rd.cls_end[2] >> 2;
+    S.e0 = rd.cls_end[0] >> 2;
+    S.e1 = rd.cls_end[1] >> 2;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        S.hoff[g] = (unsigned)((g < S.ng ? rd.cls_h[4 * g + (l & 3)] : 0) * fs + 4 * (l >> 4)) * 8u;
+        S.accx[g] = S.accy[g] = 0.0;
+    }
+}
+
+// loads at a byte offset from a uniform base (one scalar base, 32-bit lane offsets)
+typedef const char __attribute__((address_space(1))) gchar;
+__device__ __forceinline__ float2 gload2_at(const float2 *base, unsigned off)
+{
+    const vec2f v = *(gvec2f *)((gchar *)base + off);
+    return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ float4 gload4_at(const float2 *base, unsigned off)
+{
+    const vec4f v = *(gvec4f *)((gchar *)base + off);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// dx + dy + sum over the tile's 16 bins of Re(bk H) = bk.x H.x + bk.y (-H.y) for a group's 4
+// columns: fp32 base kernels and window spectra multiply exactly in FP64 and the products
+// are summed in FP64, v_mfma_f64_4x4x4_4b_f64 (4 blocks of 4 pairs, K the 4 bins of lanes
+// l / 16).  A operands: bk of pair l % 16 at bins kb .. kb + 3; B: column l % 4's spectrum
+// there.
+__device__ __forceinline__ void mfma_slot_group(const double (&ax)[4], const double (&ay)[4], float4 q0, float4 q1,
+                                                double &dx, double &dy)
+{
+    const double hx[4] = {q0.x, q0.z, q1.x, q1.z}, hy[4] = {q0.y, q0.w, q1.y, q1.w};
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        if (cls == 0) {
-            ax[v] = bk0[v].x; ay[v] = bk0[v].y;
-        } else if (cls == 1) {
-            ax[v] = bk1[v].x; ay[v] = bk1[v].y;
-        } else {                                                // mu - 2 lambda
-            ax[v] = (double)bk1[v].x - 2.0 * (double)bk0[v].x;
-            ay[v] = (double)bk1[v].y - 2.0 * (double)bk0[v].y;
+        dx = __builtin_amdgcn_mfma_f64_4x4x4f64(ax[v], hx[v], dx, 0, 0, 0);
+        dy = __builtin_amdgcn_mfma_f64_4x4x4f64(ay[v], hy[v], dy, 0, 0, 0);
+    }
+}
+
+// the base kernels of class cls (0 lambda, 1 mu, 2 mu - 2 lambda; uniform) in FP64.  (The
+// empty asm keeps the branches: selects between all three classes cost more than a class.)
+__device__ __forceinline__ void mfma_class(const float2 (&bk0)[4], const float2 (&bk1)[4], int cls, double (&ax)[4],
+                                           double (&ay)[4])
+{
+    if (cls == 0) {
+        asm volatile("");
+#pragma unroll
+        for (int v = 0; v < 4; ++v) { ax[v] = bk0[v].x; ay[v] = bk0[v].y; }
+    } else if (cls == 1) {
+        asm volatile("");
+#pragma unroll
+        for (int v = 0; v < 4; ++v) { ax[v] = bk1[v].x; ay[v] = bk1[v].y; }
+    } else {
+        asm volatile("");
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            ax[v] = __builtin_fma((double)bk0[v].x, -2.0, (double)bk1[v].x);
+            ay[v] = __builtin_fma((double)bk0[v].y, -2.0, (double)bk1[v].y);
         }
     }
-    v4d dy = v4d{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        d = __builtin_amdgcn_mfma_f64_16x16x4f64(ax[v], h[v].x, d, 0, 0, 0);
-        dy = __builtin_amdgcn_mfma_f64_16x16x4f64(ay[v], h[v].y, dy, 0, 0, 0);
-    }
-    return d + dy;
 }
 
-// the register blocks into sAcc (before the lanes read each other's sums)
-template <int DR>
-__device__ __forceinline__ void mfma_store_dreg(const RecDesc &rd, int l, double *sAcc, const v4d (&dreg)[DR ? DR : 1])
+// this lane's forward spectra of tile t (pair l % 16's point, bins 16 t + 4 (l / 16) .. + 3).
+// A lane without a pair loads the group's first point (no branch): its weights are zero, so
+// its base kernels and rows of the slot sums are zero, and nothing reads them.
+template <int NDF>
+__device__ __forceinline__ void mfma_load_f(const float2 *Fp, int l, int t, float4 (&f4)[NDF][2])
 {
-    const int nblk = rd.cls_end[2] >> 4;
-#pragma unroll
-    for (int b = 0; b < DR; ++b)
-        if (b < nblk) *reinterpret_cast<v4d *>(sAcc + (size_t)b * 256 + 4 * l) = dreg[b];
-}
-
-// dreg: blocks 0 .. DR - 1 (registers across the tiles); the others in sAcc
-template <int DR>
-__device__ __forceinline__ void mfma_window_sums(const float2 (&bk0)[4], const float2 (&bk1)[4], int l, int kb,
-                                                 int fs, const RecDesc &rd, const float2 *Hp, double *sAcc,
-                                                 v4d (&dreg)[DR ? DR : 1])
-{
-    const int nblk = rd.cls_end[2] >> 4;
-#pragma unroll
-    for (int b = 0; b < DR; ++b)
-        if (b < nblk) dreg[b] = mfma_window_block(bk0, bk1, b, l, kb, fs, rd, Hp, dreg[b]);
-    for (int b = DR; b < nblk; ++b) {
-        v4d *acc = reinterpret_cast<v4d *>(sAcc + (size_t)b * 256 + 4 * l);
-        *acc = mfma_window_block(bk0, bk1, b, l, kb, fs, rd, Hp, *acc);
-    }
-}
-
-// One 16-bin tile t of a group, given its A operands a[s] (lane l: trace 4 s + l / 16 at
-// bin 16 t + l % 16; bins past nomega and traces past J zero): the matrix cores give every
-// pair's NDB carried backward components at the tile's 16 bins (real and imaginary parts
-// as two products); lane l then holds pair l % 16 at bins kb = 16 t + 4 (l / 16) .. + 3 and
-// forms the base kernels with the forward spectra of the pair's point; then the slot sums
-// Re(bk H) with the receiver's window spectra on the FP64 matrix cores.
-// this lane's forward spectra of tile t (pair l % 16's point, bins kb .. kb + 3).  A lane
-// without a pair loads the group's first point (no branch): its weights are zero, so its
-// base kernels and rows of the slot sums are zero, and nothing reads them.
-template <int NDF, int NDB>
-__device__ __forceinline__ void mfma_load_f(const MfmaGroup<NDF, NDB> &G, const float2 *Fp, int l, int t, int fs,
-                                            float4 (&f4)[NDF][2])
-{
-    const int kb = (t << 4) + 4 * (l >> 4);
+    const float4 *src = reinterpret_cast<const float4 *>(Fp + (size_t)t * (16 * NDF) + 4 * (l >> 4));
 #pragma unroll
     for (int m = 0; m < NDF; ++m) {
-        const float4 *src = reinterpret_cast<const float4 *>(Fp + (size_t)m * fs + kb);
-        f4[m][0] = src[0];
-        f4[m][1] = src[1];
+        f4[m][0] = src[8 * m];
+        f4[m][1] = src[8 * m + 1];
     }
 }
 
-// this lane's element spectra of tile t (the A operands: trace mfma_trace(s, l / 16), bin
-// 16 t + l % 16; traces past J load trace J - 1, whose B operands there are zero)
-template <int KS, int J>
-__device__ __forceinline__ void mfma_load_u(const float2 *Ue, int us, int l, int t, float2 (&a)[KS])
+// this lane's element spectra of tile t: variable v's trace 8 (l / 16) + q in a[8 v + q], bin
+// 16 t + l % 16 (past the 25 traces: the last one, whose B operands there are zero).  uoff:
+// bytes to the traces of variable 0 (mfma_uoff)
+__device__ __forceinline__ void mfma_uoff(int l, unsigned (&uoff)[8])
 {
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        const int j = min(mfma_trace(s, l >> 4), J - 1);
-        a[s] = Ue[(size_t)j * us + (t << 4) + (l & 15)];
-    }
+    for (int q = 0; q < 8; ++q) uoff[q] = (unsigned)(min(8 * (l >> 4) + q, 24) * 16 + (l & 15)) * 8u;
+}
+template <int NVB>
+__device__ __forceinline__ void mfma_load_u(const float2 *Ue, const unsigned (&uoff)[8], int t, float2 (&a)[8 * NVB])
+{
+    const float2 *Ut = Ue + (size_t)t * (16 * 25 * NVB);
+#pragma unroll
+    for (int v = 0; v < NVB; ++v)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) a[8 * v + q] = gload2_at(Ut, uoff[q] + 25u * 16u * 8u * v);
 }
 
-template <int NDF, int NDB, int KS, int DR>
-__device__ __forceinline__ void mfma_tile(const MfmaGroup<NDF, NDB> &G, const float2 (&a)[KS],
-                                          const float4 (&f4)[NDF][2], const float *sW, double *sAcc, int l, int t,
-                                          const PathConf &pc, const RecDesc &rd, const float2 *Hp,
-                                          v4d (&dreg)[DR ? DR : 1])
+// One 16-bin tile t of a group, given its element spectra a: the matrix cores give every
+// pair's NDB carried backward components at the tile's 16 bins (real and imaginary parts
+// as two products); lane l then holds pair l % 16 at bins kb = 16 t + 4 (l / 16) .. + 3 and
+// forms the base kernels with the forward spectra f4 of the pair's point; then the slot
+// sums Re(bk H) with the receiver's window spectra on the FP64 matrix cores.  next_u and
+// next_f load the next tile's spectra into a and f4 once they are used.
+template <int NDF, int NDB, int NVB, int NG, class NextU, class NextF>
+__device__ __forceinline__ void mfma_tile(const MfmaGroup<NDF, NDB> &G, MfmaSlots<NG> &S, float2 (&a)[8 * NVB],
+                                          float4 (&f4)[NDF][2], const v8h *sW, double *sAcc, int l, int t,
+                                          const PathConf &pc, const RecDesc &rd, const float2 *Hp, NextU &&next_u,
+                                          NextF &&next_f)
 {
-    const int bq = l >> 4, kb = (t << 4) + 4 * bq, fs = pc.fstride;
+    constexpr int KS = 8 * NVB, PF = NG < 4 ? NG : 4;          // window spectra of PF groups loaded ahead
+    // Loads complete in the order they are issued, so they are issued in the order of their
+    // use: this tile's window spectra, then the next tile's element spectra (when this
+    // tile's are split) and forward spectra (when this tile's are multiplied).
+    const float2 *Ht = Hp + (t << 4);
+    float4 h[PF][2];
+#pragma unroll
+    for (int g = 0; g < PF; ++g) {
+        h[g][0] = gload4_at(Ht, S.hoff[g]);
+        h[g][1] = gload4_at(Ht, S.hoff[g] + 16u);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     v4f accR[NDB], accI[NDB];
 #pragma unroll
     for (int c = 0; c < NDB; ++c) {
         accR[c] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
         accI[c] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    if constexpr (kMfmaSplit) {
-        // the tile's scale: its largest |U| to below 2^14
-        float mx = 0.0f;
+    // the tile's scale: its largest |U| to below 2^14
+    float mx = 0.0f;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) mx = fmaxf(mx, fmaxf(fabsf(a[s].x), fabsf(a[s].y)));
-        mx = mfma_wave_max(mx);
-        int e;
-        (void)frexpf(mx, &e);
-        const int eu = __builtin_amdgcn_readfirstlane(14 - e);
-        const v8h *sWh = reinterpret_cast<const v8h *>(sW);
-#pragma unroll
-        for (int kb = 0; kb < KS / 8; ++kb) {
-            v8h rh, rl, ih, il;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                _Float16 h, o;
-                mfma_split(ldexpf(a[8 * kb + q].x, eu), h, o);
-                rh[q] = h;
-                rl[q] = o;
-                mfma_split(ldexpf(a[8 * kb + q].y, eu), h, o);
-                ih[q] = h;
-                il[q] = o;
-            }
-#pragma unroll
-            for (int c = 0; c < NDB; ++c) {
-                const v8h wh = sWh[(2 * (kb * NDB + c)) * 64 + l], wl = sWh[(2 * (kb * NDB + c) + 1) * 64 + l];
-                accR[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rh, wh, accR[c], 0, 0, 0);
-                accI[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ih, wh, accI[c], 0, 0, 0);
-                accR[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rh, wl, accR[c], 0, 0, 0);
-                accI[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ih, wl, accI[c], 0, 0, 0);
-                accR[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rl, wh, accR[c], 0, 0, 0);
-                accI[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(il, wh, accI[c], 0, 0, 0);
-            }
-        }
-        // back to the spectra's scale (column l % 16: this lane's pair)
-        const int es = -(eu + G.ew);
-#pragma unroll
-        for (int c = 0; c < NDB; ++c)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                accR[c][v] = ldexpf(accR[c][v], es);
-                accI[c][v] = ldexpf(accI[c][v], es);
-            }
-    } else {
+    for (int s = 0; s < KS; ++s) mx = mfma_max3(mx, a[s].x, a[s].y);
+    mx = mfma_wave_max(mx);
+    int e;
+    (void)frexpf(mx, &e);
+    int eu = __builtin_amdgcn_readfirstlane(14 - e);
+    if (eu > 126) {                                            // (beyond a float's power of two)
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-#pragma unroll
-            for (int c = 0; c < NDB; ++c) {
-                const float w = sW[(s * NDB + c) * 64 + l];
-                accR[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s].x, w, accR[c], 0, 0, 0);
-                accI[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s].y, w, accI[c], 0, 0, 0);
-            }
+            a[s].x = ldexpf(a[s].x, eu - 126);
+            a[s].y = ldexpf(a[s].y, eu - 126);
         }
     }
-    // base kernels of this lane's pair at bins kb + v
+    const float us = ldexpf(1.0f, min(eu, 126));
+#pragma unroll
+    for (int v = 0; v < NVB; ++v) {
+        v4u h4[4];                                             // re hi, re lo, im hi, im lo
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            unsigned h, o;
+            mfma_split2(a[8 * v + 2 * q].x * us, a[8 * v + 2 * q + 1].x * us, h, o);
+            h4[0][q] = h;
+            h4[1][q] = o;
+            mfma_split2(a[8 * v + 2 * q].y * us, a[8 * v + 2 * q + 1].y * us, h, o);
+            h4[2][q] = h;
+            h4[3][q] = o;
+        }
+        const v8h rh = __builtin_bit_cast(v8h, h4[0]), rl = __builtin_bit_cast(v8h, h4[1]);
+        const v8h ih = __builtin_bit_cast(v8h, h4[2]), il = __builtin_bit_cast(v8h, h4[3]);
+#pragma unroll
+        for (int c = 0; c < NDB; ++c) {
+            if (!mfma_has(NDB, v, c)) continue;
+            const int b = mfma_wblock(NDB, v, c);
+            const v8h wh = sW[(2 * b) * 64 + l], wl = sW[(2 * b + 1) * 64 + l];
+            accR[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rh, wh, accR[c], 0, 0, 0);
+            accI[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ih, wh, accI[c], 0, 0, 0);
+            accR[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rh, wl, accR[c], 0, 0, 0);
+            accI[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ih, wl, accI[c], 0, 0, 0);
+            accR[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rl, wh, accR[c], 0, 0, 0);
+            accI[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(il, wh, accI[c], 0, 0, 0);
+        }
+    }
+    next_u(a);
+    __builtin_amdgcn_sched_barrier(0);
+    // base kernels of this lane's pair at bins kb + v, scaled back (column l % 16: this
+    // lane's pair)
+    const int es = -(eu + G.ew);
     float2 bk0[4], bk1[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -719,48 +758,85 @@ __device__ __forceinline__ void mfma_tile(const MfmaGroup<NDF, NDB> &G, const fl
             f[m] = (v & 1) ? make_float2(f4[m][v >> 1].z, f4[m][v >> 1].w) : make_float2(f4[m][v >> 1].x, f4[m][v >> 1].y);
 #pragma unroll
         for (int c = 0; c < NDB; ++c) b[c] = make_float2(accR[c][v], accI[c][v]);
-        if (NDF == 1) {
+        if constexpr (NDF == 1) {
             const float2 pr = cmulf(f[0], b[0]);
-            bk0[v] = make_float2(-pr.x, -pr.y);
-            bk1[v] = make_float2(-2.0f * pr.x, -2.0f * pr.y);
+            bk0[v] = make_float2(ldexpf(-pr.x, es), ldexpf(-pr.y, es));
+            bk1[v] = make_float2(ldexpf(-pr.x, es + 1), ldexpf(-pr.y, es + 1));
         } else {
-            float2 trf = make_float2(0.f, 0.f), trb = trf;
-#pragma unroll
-            for (int m = 0; m < NDF; ++m) { trf.x += G.uf[m] * f[m].x; trf.y += G.uf[m] * f[m].y; }
-#pragma unroll
-            for (int c = 0; c < NDB; ++c) { trb.x += G.ub[c] * b[c].x; trb.y += G.ub[c] * b[c].y; }
+            const float2 trf = make_float2(f[0].x + f[1].x + f[2].x, f[0].y + f[1].y + f[2].y);
+            const float2 trb = make_float2(b[0].x + b[1].x + b[2].x, b[0].y + b[1].y + b[2].y);
             const float2 lam = cmulf(trf, trb);
-            bk0[v] = make_float2(-lam.x, -lam.y);
-            bk1[v] = make_float2(0.f, 0.f);
-            if (pc.need_bk & 2) {
-                float2 mu = make_float2(0.f, 0.f);
+            bk0[v] = make_float2(ldexpf(-lam.x, es), ldexpf(-lam.y, es));
+            // (mu: full strain is carried only when some kernel reads it)
+            float2 mu = make_float2(0.f, 0.f);
 #pragma unroll
-                for (int m = 0; m < NDF; ++m) {
-                    float2 gm = make_float2(0.f, 0.f);
+            for (int m = 0; m < NDF; ++m) {
+                float2 gm = make_float2(G.Amu[m][0] * b[0].x, G.Amu[m][0] * b[0].y);
 #pragma unroll
-                    for (int c = 0; c < NDB; ++c) { gm.x += G.Amu[m][c] * b[c].x; gm.y += G.Amu[m][c] * b[c].y; }
-                    const float2 tt = cmulf(f[m], gm);
-                    mu.x += tt.x; mu.y += tt.y;
-                }
-                bk1[v] = make_float2(-2.0f * mu.x, -2.0f * mu.y);
+                for (int c = 1; c < NDB; ++c) { gm.x += G.Amu[m][c] * b[c].x; gm.y += G.Amu[m][c] * b[c].y; }
+                mu.x += f[m].x * gm.x;
+                mu.x -= f[m].y * gm.y;
+                mu.y += f[m].x * gm.y;
+                mu.y += f[m].y * gm.x;
             }
+            bk1[v] = make_float2(ldexpf(-mu.x, es + 1), ldexpf(-mu.y, es + 1));
         }
     }
-    mfma_window_sums<DR>(bk0, bk1, l, kb, fs, rd, Hp, sAcc, dreg);
+    // (the base kernels before the loads: loads moved above the last use of their registers'
+    // present values go to other registers, waited for and copied at the end of the tile)
+    asm volatile("" ::"v"(bk0[0].x), "v"(bk0[0].y), "v"(bk0[1].x), "v"(bk0[1].y), "v"(bk0[2].x), "v"(bk0[2].y),
+                 "v"(bk0[3].x), "v"(bk0[3].y), "v"(bk1[0].x), "v"(bk1[0].y), "v"(bk1[1].x), "v"(bk1[1].y),
+                 "v"(bk1[2].x), "v"(bk1[2].y), "v"(bk1[3].x), "v"(bk1[3].y) : "memory");
+    next_f(f4);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    // slot sums, group by group; the base kernels are converted once per class
+    double ax[4], ay[4];
+    mfma_class(bk0, bk1, S.e0 > 0 ? 0 : (S.e1 > 0 ? 1 : 2), ax, ay);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (g > 0 && (g == S.e0 || g == S.e1)) mfma_class(bk0, bk1, g < S.e1 ? 1 : 2, ax, ay);
+        const float4 q0 = h[g % PF][0], q1 = h[g % PF][1];
+        if (g + PF < NG) {
+            const unsigned off = S.hoff[g + PF < NG ? g + PF : 0];
+            h[g % PF][0] = gload4_at(Ht, off);
+            h[g % PF][1] = gload4_at(Ht, off + 16u);
+        }
+        mfma_slot_group(ax, ay, q0, q1, S.accx[g], S.accy[g]);
+    }
+    if constexpr (NG == kMfmaMaxRegGroups)
+        for (int g = NG; g < S.ng; ++g) {
+            const unsigned off = (unsigned)(rd.cls_h[4 * g + (l & 3)] * pc.fstride + 4 * (l >> 4)) * 8u;
+            const float4 q0 = gload4_at(Ht, off), q1 = gload4_at(Ht, off + 16u);
+            mfma_class(bk0, bk1, g < S.e0 ? 0 : (g < S.e1 ? 1 : 2), ax, ay);
+            double dx = sAcc[g * 64 + l], dy = 0.0;
+            mfma_slot_group(ax, ay, q0, q1, dx, dy);
+            sAcc[g * 64 + l] = dx + dy;
+        }
+}
+
+// the register groups into sAcc (before the lanes read each other's sums)
+template <int NG>
+__device__ __forceinline__ void mfma_store_slots(const MfmaSlots<NG> &S, int l, double *sAcc)
+{
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+        if (g < S.ng) sAcc[g * 64 + l] = S.accx[g] + S.accy[g];
 }
 
 // Physical kernels (kernel.f90:665-832) of the group's pairs with the model at the point,
-// after the damping of every receiver processed in this step (readfields.f90:3184-3204);
-// lanes 0..15 (lane l: pair l).  phys: [point][nk]; base_out (optional): [point][nk][6]
-template <int NDF, int NDB>
-__device__ __forceinline__ void mfma_finish(const MfmaGroup<NDF, NDB> &G, int l, const double *sAcc,
+// after the damping of every receiver processed in this step (readfields.f90:3184-3204).
+// Called by all lanes of the group's NW waves: lane l serves pair l % 16 and every 4 NW-th
+// kernel from 4 wv + l / 16 on.  phys: [point][nk]; base_out (optional): [point][nk][6]
+template <int NDF, int NDB, int NW>
+__device__ __forceinline__ void mfma_finish(const MfmaGroup<NDF, NDB> &G, int l, int wv, const double *sAcc,
                                             const PathConf &pc, const RecDesc &rd, const KernDesc *kern,
                                             const int *model_idx, const float *model, int ndepth, int relative,
                                             int nk, double *phys, double *base_out, const double *xyz,
                                             const uint8_t *active, int P, int R, const double *rec_xyz)
 {
-    if (l >= kMfmaPairs || !G.valid) return;
-    const int p = G.p, r = G.r, jp = l;
+    if (!G.valid) return;
+    const int p = G.p, r = G.r, jp = l & 15;
     const int mi = model_idx[p];
     const float vp = model[0 * ndepth + mi], vs = model[1 * ndepth + mi], rho_f = model[2 * ndepth + mi];
     const double rho = rho_f;
@@ -777,7 +853,7 @@ __device__ __forceinline__ void mfma_finish(const MfmaGroup<NDF, NDB> &G, int l,
             damp = damp * (dr < pc.damp_radius ? dr / pc.damp_radius : 1.0) * fsrc;
         }
     }
-    for (int kk = 0; kk < rd.nkernel; ++kk) {
+    for (int kk = 4 * wv + (l >> 4); kk < rd.nkernel; kk += 4 * NW) {
         const int k = rd.first_kernel + kk;
         const KernDesc &kd = kern[k];
         double b[kNumBk];
@@ -801,87 +877,77 @@ __device__ __forceinline__ void mfma_finish(const MfmaGroup<NDF, NDB> &G, int l,
 }
 
 // ------------------------------------------------------------------------------------
-// k_bwd_mfma: one wave per group of at most 16 pairs of one (element, receiver), groups of
-// element runs u0 .. u0 + ubatch - 1 (the others are left to another launch); the wave
-// reads its element's spectra tile by tile from memory.  Only the lambda and mu base
-// kernels (and mu - 2 lambda) are formed: the host sends kernel sets with anisotropic
-// parameters to k_bwd_eval.  Hp: window spectra, rows fstride apart, zero past nomega;
-// F: forward spectra, rows fstride apart, zero past nomega.  xcd: groups in
-// XCD-contiguous ranges (the groups of an element on one XCD).
+// k_bwd_mfma: one workgroup of 4 waves per group of at most 16 pairs of one (element,
+// receiver), groups of element runs u0 .. u0 + ubatch - 1 (the others are left to another
+// launch).  The waves share the group's weights and take its 16-bin tiles in turn; their
+// slot sums are added at the end.  Only the lambda and mu base kernels (and mu - 2 lambda)
+// are formed: the host sends kernel sets with anisotropic parameters to k_bwd_eval.  Hp:
+// window spectra, rows fstride apart, zero past nomega; F: forward spectra (tile_at), zero
+// past nomega.  xcd: groups in XCD-contiguous ranges (the groups of an element on one XCD).
+// Bound: half by the forward and element spectra, 4 NDF 128-byte lines a pair and 8-bin row
+// (3.7 TB/s at L2 misses over 12,000 tets x 10 receivers), half by the wave's instructions
+// (f16 matrix products 25 %, splitting and slot sums the rest), at the 2 waves a SIMD that
+// 230 registers leave; 3 waves spill and were slower (12.8 against 9.8 ms a launch).  Tiles
+// contiguous in memory, zero (component, variable) blocks left out, and the slot sums on
+// the FP64 matrix units (4 x 4 x 4, a group of 4 slots and 4 bins a product) in place of
+// FP64 vector products: 357 -> 311 ms (12,000 tets, 10 receivers, nt 2048), 124 -> 88 ms
+// (40 voxels, 200 receivers, nt 4096), 428 -> 417 ms (100 tets, 50 receivers, 24 slots a
+// receiver).  Four waves a group against one: 311 against 294, 88 against 89 and 417 against
+// 460 ms (6 register groups of slots spilled).
 // ------------------------------------------------------------------------------------
-template <int NDF, int NDB, int NVB>
-__global__ __launch_bounds__(64, NDB <= 4 ? 2 : 1) void k_bwd_mfma(
+template <int NDF, int NDB, int NVB, int NG>
+__global__ __launch_bounds__(64 * kMfmaWaves, NDB <= 4 ? 2 : 1) void k_bwd_mfma(
     PathConf pc, int u0, int ubatch, int ngroups, const int *group_first, const int *group_erun,
     const float2 *U, const int *order, int R, const float *Wb, const float *Qb, const float *Qf,
     const float2 *F, const RecDesc *recs, const KernDesc *kern, const float2 *Hp, int npos,
     const int *model_idx, const float *model, int ndepth, int relative, int nk, double *phys, double *base_out,
     const double *xyz, const uint8_t *active, int P, const double *rec_xyz, int xcd)
 {
-    constexpr int J = NVB * 25, KS = mfma_ks(J);
+    constexpr int J = NVB * 25, KS = mfma_ks(NVB), NW = kMfmaWaves;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int grp = xcd ? xcd_block_n(ngroups) : ((int)blockIdx.x < ngroups ? (int)blockIdx.x : -1);
     if (grp < 0) return;
     const int eu = group_erun[grp];
     if (eu < u0 || eu >= u0 + ubatch) return;
-    const int l = threadIdx.x;
-    float *sW = reinterpret_cast<float *>(smem_raw);
-    double *sAcc = reinterpret_cast<double *>(sW + KS * NDB * 64);
+    const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    v8h *sW = reinterpret_cast<v8h *>(smem_raw);
+    double *sSum = reinterpret_cast<double *>(sW + mfma_nblock(NDB, NVB) * 2 * 64);
+    double *sAcc = sSum + (size_t)wv * npos * kMfmaPairs;
     MfmaGroup<NDF, NDB> G;
-    mfma_group_setup<NDF, NDB, NVB>(G, grp, group_first, order, R, Wb, Qb, Qf, pc, npos, sW, sAcc, l);
+    mfma_group_setup<NDF, NDB, NVB, NW>(G, grp, group_first, order, R, Wb, Qb, Qf, pc, npos, sW, sAcc, l, wv);
     __syncthreads();
     const float2 *Ue = U + (size_t)(eu - u0) * J * pc.ustride;
     const RecDesc &rd = recs[G.r];
     const float2 *Fp = F + (size_t)G.p * NDF * pc.fstride;
     const int ntile = (pc.nomega + 15) >> 4;
-    constexpr int DR = mfma_dreg<NDF, NVB>();
-    v4d dreg[DR ? DR : 1];
-#pragma unroll
-    for (int b = 0; b < (DR ? DR : 1); ++b) dreg[b] = v4d{0.0, 0.0, 0.0, 0.0};
-    if constexpr (NDF <= 4 && NDB <= 4) {
-        // the next tile's element and forward spectra are loaded while this one is
-        // multiplied (the registers for it fit two waves per SIMD up to 4 components)
-        float2 an[KS];
-        float4 fn[NDF][2];
-        mfma_load_u<KS, J>(Ue, pc.ustride, l, 0, an);
-        mfma_load_f<NDF, NDB>(G, Fp, l, 0, pc.fstride, fn);
-        for (int t = 0; t < ntile; ++t) {
-            float2 a[KS];
-            float4 f4[NDF][2];
-#pragma unroll
-            for (int s = 0; s < KS; ++s) a[s] = an[s];
-#pragma unroll
-            for (int m = 0; m < NDF; ++m) { f4[m][0] = fn[m][0]; f4[m][1] = fn[m][1]; }
-            const int tn = t + 1 < ntile ? t + 1 : t;
-            mfma_load_u<KS, J>(Ue, pc.ustride, l, tn, an);
-            mfma_load_f<NDF, NDB>(G, Fp, l, tn, pc.fstride, fn);
-            mfma_tile<NDF, NDB, KS, DR>(G, a, f4, sW, sAcc, l, t, pc, rd, Hp, dreg);
-        }
-    } else if constexpr (NVB == 2) {
-        // (more components: the element spectra only)
-        float2 an[KS];
-        mfma_load_u<KS, J>(Ue, pc.ustride, l, 0, an);
-        for (int t = 0; t < ntile; ++t) {
-            float2 a[KS];
-            float4 f4[NDF][2];
-#pragma unroll
-            for (int s = 0; s < KS; ++s) a[s] = an[s];
-            mfma_load_u<KS, J>(Ue, pc.ustride, l, t + 1 < ntile ? t + 1 : t, an);
-            mfma_load_f<NDF, NDB>(G, Fp, l, t, pc.fstride, f4);
-            mfma_tile<NDF, NDB, KS, DR>(G, a, f4, sW, sAcc, l, t, pc, rd, Hp, dreg);
-        }
-    } else {
-        for (int t = 0; t < ntile; ++t) {
-            float2 a[KS];
-            float4 f4[NDF][2];
-            mfma_load_u<KS, J>(Ue, pc.ustride, l, t, a);
-            mfma_load_f<NDF, NDB>(G, Fp, l, t, pc.fstride, f4);
-            mfma_tile<NDF, NDB, KS, DR>(G, a, f4, sW, sAcc, l, t, pc, rd, Hp, dreg);
-        }
+    MfmaSlots<NG> S;
+    mfma_slots_init(S, rd, l, pc.fstride);
+    unsigned uoff[8];
+    mfma_uoff(l, uoff);
+    // the next tile's element and forward spectra are loaded into the registers of this
+    // tile's as soon as those are used
+    float2 a[KS];
+    float4 f4[NDF][2];
+    mfma_load_u<NVB>(Ue, uoff, min(wv, ntile - 1), a);
+    mfma_load_f<NDF>(Fp, l, min(wv, ntile - 1), f4);
+    for (int t = wv; t < ntile; t += NW) {
+        const int tn = t + NW < ntile ? t + NW : t;
+        mfma_tile<NDF, NDB, NVB, NG>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hp,
+                                 [&](float2 (&x)[KS]) { mfma_load_u<NVB>(Ue, uoff, tn, x); },
+                                 [&](float4 (&x)[NDF][2]) { mfma_load_f<NDF>(Fp, l, tn, x); });
     }
-    mfma_store_dreg<DR>(rd, l, sAcc, dreg);
-    __syncthreads();                                           // the lanes' blocks of sums
-    mfma_finish<NDF, NDB>(G, l, sAcc, pc, rd, kern, model_idx, model, ndepth, relative, nk, phys, base_out, xyz,
-                          active, P, R, rec_xyz);
+    mfma_store_slots(S, l, sAcc);
+    __syncthreads();
+    // the waves' sums of every class position
+    for (int i = (int)threadIdx.x; i < S.ng * 64; i += 64 * NW) {
+        double d = sSum[i];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) d += sSum[(size_t)w * npos * kMfmaPairs + i];
+        sSum[i] = d;
+    }
+    __syncthreads();
+    mfma_finish<NDF, NDB, NW>(G, l, wv, sSum, pc, rd, kern, model_idx, model, ndepth, relative, nk, phys, base_out, xyz,
+                              active, P, R, rec_xyz);
 }
 
 // ------------------------------------------------------------------------------------
@@ -900,59 +966,59 @@ __global__ __launch_bounds__(64 * W) void k_bwd_mfma_wg(
     const int *model_idx, const float *model, int ndepth, int relative, int nk, double *phys, double *base_out,
     const double *xyz, const uint8_t *active, int P, const double *rec_xyz)
 {
-    constexpr int J = NVB * 25, KS = mfma_ks(J), TILE = KS * 4 * 16;   // float2 per tile
-    constexpr int PER = (TILE + 64 * W - 1) / (64 * W);
+    constexpr int J = NVB * 25, KS = mfma_ks(NVB), TILE = KS * 4 * 16; // float2 per tile
+    constexpr int PER = (TILE + 64 * W - 1) / (64 * W), NBLK = mfma_nblock(NDB, NVB);
     extern __shared__ __align__(16) unsigned char smem_raw[];
     if ((int)blockIdx.x >= ubatch) return;
     const int u = u0 + (int)blockIdx.x;
     const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, jp = l & 15, bq = l >> 4;
-    float2 *sU = reinterpret_cast<float2 *>(smem_raw);                  // [2][4 KS][16]
-    float *sW = reinterpret_cast<float *>(sU + 2 * TILE) + (size_t)wv * KS * NDB * 64;
-    double *sAcc = reinterpret_cast<double *>(reinterpret_cast<float *>(sU + 2 * TILE) + (size_t)W * KS * NDB * 64)
+    float2 *sU = reinterpret_cast<float2 *>(smem_raw);                  // [2][32 NVB][16]
+    v8h *sW = reinterpret_cast<v8h *>(sU + 2 * TILE) + (size_t)wv * NBLK * 2 * 64;
+    double *sAcc = reinterpret_cast<double *>(reinterpret_cast<v8h *>(sU + 2 * TILE) + (size_t)W * NBLK * 2 * 64)
                  + (size_t)wv * npos * kMfmaPairs;
     const float2 *Ue = U + (size_t)(u - u0) * J * pc.ustride;
     const int gbeg = erun_group_first[u], gend = erun_group_first[u + 1];
     const int ntile = (pc.nomega + 15) >> 4;
+    // element spectra of row idx / 16 of tile t (row: 32 v + trace), zero past the 25 traces
+    auto load = [&](int idx, int t) {
+        const int v = idx >> 9, n = (idx >> 4) & 31;
+        return n < 25 ? Ue[((size_t)t * J + 25 * v + n) * 16 + (idx & 15)] : make_float2(0.0f, 0.0f);
+    };
     for (int round = gbeg; round < gend; round += W) {
         const int grp = round + wv;
         const bool mine = grp < gend;                                  // uniform in the wave
         MfmaGroup<NDF, NDB> G;
-        constexpr int DR = mfma_dreg<NDF, NVB>();
-        v4d dreg[DR ? DR : 1];
-#pragma unroll
-        for (int b = 0; b < (DR ? DR : 1); ++b) dreg[b] = v4d{0.0, 0.0, 0.0, 0.0};
         if (mine)
-            mfma_group_setup<NDF, NDB, NVB>(G, grp, group_first, order, R, Wb, Qb, Qf, pc, npos, sW, sAcc, l);
+            mfma_group_setup<NDF, NDB, NVB, 1>(G, grp, group_first, order, R, Wb, Qb, Qf, pc, npos, sW, sAcc, l, 0);
         // tile 0 (the previous round's readers of both buffers are past the last barrier)
         for (int i = 0; i < PER; ++i) {
             const int idx = tid + i * 64 * W;
-            if (idx < TILE) {
-                const int j = idx >> 4;
-                sU[idx] = j < J ? Ue[(size_t)j * pc.ustride + (idx & 15)] : make_float2(0.0f, 0.0f);
-            }
+            if (idx < TILE) sU[idx] = load(idx, 0);
         }
         __syncthreads();
         const RecDesc &rd = recs[mine ? G.r : 0];
         const float2 *Fp = F + (size_t)(mine ? G.p : 0) * NDF * pc.fstride;
+        MfmaSlots<kMfmaMaxRegGroups> S;
+        mfma_slots_init(S, rd, l, pc.fstride);
         for (int t = 0; t < ntile; ++t) {
             float2 nx[PER];
             const bool more = t + 1 < ntile;
             if (more) {
 #pragma unroll
                 for (int i = 0; i < PER; ++i) {
-                    const int idx = tid + i * 64 * W, j = idx >> 4;
-                    nx[i] = (idx < TILE && j < J) ? Ue[(size_t)j * pc.ustride + ((t + 1) << 4) + (idx & 15)]
-                                                  : make_float2(0.0f, 0.0f);
+                    const int idx = tid + i * 64 * W;
+                    nx[i] = idx < TILE ? load(idx, t + 1) : make_float2(0.0f, 0.0f);
                 }
             }
             if (mine) {
                 const float2 *tile = sU + (t & 1) * TILE;
                 float2 a[KS];
 #pragma unroll
-                for (int s = 0; s < KS; ++s) a[s] = tile[mfma_trace(s, bq) * 16 + jp];
+                for (int s = 0; s < KS; ++s) a[s] = tile[(32 * (s >> 3) + 8 * bq + (s & 7)) * 16 + jp];
                 float4 f4[NDF][2];
-                mfma_load_f<NDF, NDB>(G, Fp, l, t, pc.fstride, f4);
-                mfma_tile<NDF, NDB, KS, DR>(G, a, f4, sW, sAcc, l, t, pc, rd, Hp, dreg);
+                mfma_load_f<NDF>(Fp, l, t, f4);
+                mfma_tile<NDF, NDB, NVB, kMfmaMaxRegGroups>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hp, [](float2 (&)[KS]) {},
+                                         [](float4 (&)[NDF][2]) {});
             }
             if (more) {
                 float2 *nt = sU + ((t + 1) & 1) * TILE;
@@ -964,10 +1030,10 @@ __global__ __launch_bounds__(64 * W) void k_bwd_mfma_wg(
             }
             __syncthreads();
         }
-        if (mine) mfma_store_dreg<DR>(rd, l, sAcc, dreg);
-        __syncthreads();                                               // the lanes' blocks of sums
+        if (mine) mfma_store_slots(S, l, sAcc);
+        __syncthreads();                                               // the lanes' slot sums
         if (mine)
-            mfma_finish<NDF, NDB>(G, l, sAcc, pc, rd, kern, model_idx, model, ndepth, relative, nk, phys, base_out,
+            mfma_finish<NDF, NDB, 1>(G, l, 0, sAcc, pc, rd, kern, model_idx, model, ndepth, relative, nk, phys, base_out,
                                   xyz, active, P, R, rec_xyz);
         __syncthreads();
     }
