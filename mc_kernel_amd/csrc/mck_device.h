@@ -116,10 +116,16 @@ __host__ __device__ constexpr size_t tile_at(int n, int c, int k) { return ((siz
 
 // LDS layout of the per-point operator set-up
 struct OpShared {
-    double invj[25][4];     // [ipol + 5 jpol]
+    union {
+        double invj[25][4];     // [ipol + 5 jpol]
+        double D[3][25];        // d/ds, d/dz and 1/s at the point by node (op_weights)
+    };
     double sinv[25];        // 1 / s at the nodes
     double li[5], lj[5];
-    double M[6][kMaxSim][6];// output comp x simulation x strain comp
+    union {
+        double M[6][kMaxSim][6];// output comp x simulation x strain comp
+        double cf[6 * kMaxVar][3];  // coefficients of D by (comp, variable) (op_weights)
+    };
     float Q[6][6];          // earth Voigt component x carried component (source mode)
     int elem;
     int axial;

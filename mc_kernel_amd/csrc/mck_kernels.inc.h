@@ -887,8 +887,8 @@ __global__ void k_elem_tables(DevDb db, double *out)
 // The set-up runs in two parts separated by a barrier: op_setup_parts (element tables,
 // Lagrange bases, output transform) and op_weights.  nthr threads cooperate (tid < nthr);
 // threads role_l .. role_l + 9 form the ten Lagrange basis values, role_xf .. role_xf +
-// nd - 1 the rotation columns and role_m .. role_m + nsim - 1 the output transform of one
-// simulation each (each value is computed exactly as by a single thread).
+// nd - 1 the rotation columns and role_m .. role_m + 6 nsim - 1 the output transform of one
+// strain component of a simulation each.
 __device__ void op_setup_parts(OpShared &S, const DevDb &db, const PathConf &pc, const DevFrame &fr,
                                const Located &L, bool fwd, int nd, const int *comps, bool src_mode,
                                int tid, int nthr, int role_l, int role_xf, int role_m)
@@ -908,11 +908,13 @@ __device__ void op_setup_parts(OpShared &S, const DevDb &db, const PathConf &pc,
         const int i = is_xi ? which : which - 5;
         const double *pts = is_xi ? (db.axis[e] ? c_basis.glj : c_basis.gll) : c_basis.gll;
         const double x = is_xi ? L.xi : L.eta;
-        double v = 1.0;
+        double v = 1.0, d = 1.0;
         for (int m = 0; m < 5; ++m) {
             if (m == i) continue;
-            v = v * (x - pts[m]) / (pts[i] - pts[m]);
+            v *= x - pts[m];
+            d *= pts[i] - pts[m];
         }
+        v /= d;
         if (is_xi) S.li[i] = v; else S.lj[i] = v;
     }
     if (pc.full && src_mode && tid >= role_xf && tid < role_xf + nd) {
@@ -926,57 +928,55 @@ __device__ void op_setup_parts(OpShared &S, const DevDb &db, const PathConf &pc,
         for (int i = 0; i < 6; ++i) S.Q[i][c] = (float)t[i];
     }
     const int nsim = fwd ? pc.nsim_fwd : 1;
-    if (tid >= role_m && tid < role_m + nsim) {
-        // output transform of simulation si: sign flip of comps 4, 6 (readfields.f90:
-        // 2180-2184), azimuthal factors, 1/amplitude (and, in earth mode, the rotations)
-        const int si = tid - role_m;
-        const double amp = db.amplitude;
-        double az[6];
+    if (tid >= role_m && tid < role_m + 6 * nsim) {
+        // output transform of strain component m of simulation si: sign flip of comps 4, 6
+        // (readfields.f90:2180-2184), azimuthal factors, 1/amplitude (and, in earth mode,
+        // the rotations)
+        const int si = (tid - role_m) / 6, m = tid - role_m - 6 * si;
+        double az = 1.0;
         if (fwd) {
-            int isim = pc.fwd_sim[si];
-            double a1 = azim_factor(L.phi, pc.mij, isim, 1), a2 = azim_factor(L.phi, pc.mij, isim, 2);
-            az[0] = a1; az[1] = a1; az[2] = a1; az[3] = a2; az[4] = a1; az[5] = a2;
-        } else if (pc.bwd_isim == 1) {
-            for (int m = 0; m < 6; ++m) az[m] = 1.0;
-        } else {
-            double a1 = pc.bwd_fi[1] * cos(L.phi) + pc.bwd_fi[2] * sin(L.phi);
-            double a2 = -pc.bwd_fi[1] * sin(L.phi) + pc.bwd_fi[2] * cos(L.phi);
-            az[0] = a1; az[1] = a1; az[2] = a1; az[3] = a2; az[4] = a1 * 2; az[5] = a2 * 2;
-        }
-        if (!pc.full) {
-            for (int m = 0; m < 6; ++m) S.M[0][si][m] = (m == 0) ? az[0] / amp : 0.0;
-        } else if (src_mode) {
-            for (int c = 0; c < 6; ++c)
-                for (int m = 0; m < 6; ++m)
-                    S.M[c][si][m] = (c < nd && m == comps[c])
-                                  ? ((m == 3 || m == 5) ? -1.0 : 1.0) * az[m] / amp : 0.0;
-        } else {
+            az = azim_factor(L.phi, pc.mij, pc.fwd_sim[si], (m == 3 || m == 5) ? 2 : 1);
+        } else if (pc.bwd_isim != 1) {
             const double sp = sin(L.phi), cp = cos(L.phi);
-            for (int m = 0; m < 6; ++m) {
-                double t[6] = {0, 0, 0, 0, 0, 0};
-                t[m] = 1.0;
-                rot_src_to_xyz(t, sp, cp);
-                rot_xyz_to_earth(t, fr.sin_lon, fr.cos_lon, fr.sin_colat, fr.cos_colat);
-                double f = ((m == 3 || m == 5) ? -1.0 : 1.0) * az[m] / amp;
-                for (int c = 0; c < 6; ++c) S.M[c][si][m] = t[c] * f;
-            }
+            az = (m == 3 || m == 5) ? -pc.bwd_fi[1] * sp + pc.bwd_fi[2] * cp
+                                    : pc.bwd_fi[1] * cp + pc.bwd_fi[2] * sp;
+            if (m >= 4) az *= 2;
+        }
+        const double f = az / db.amplitude, sf = (m == 3 || m == 5) ? -f : f;
+        if (!pc.full) {
+            S.M[0][si][m] = (m == 0) ? f : 0.0;
+        } else if (src_mode) {
+            for (int c = 0; c < 6; ++c) S.M[c][si][m] = (c < nd && m == comps[c]) ? sf : 0.0;
+        } else {
+            double t[6] = {0, 0, 0, 0, 0, 0};
+            t[m] = 1.0;
+            rot_src_to_xyz(t, sin(L.phi), cos(L.phi));
+            rot_xyz_to_earth(t, fr.sin_lon, fr.cos_lon, fr.sin_colat, fr.cos_colat);
+            for (int c = 0; c < 6; ++c) S.M[c][si][m] = t[c] * sf;
         }
     }
 }
 
 // W[(c * nvar + v) * 25 + node] from the tables of op_setup_parts (W: LDS or global,
-// f32 for the spectra kernels, f64 for the seismograms)
-template <class T>
-__device__ void op_weights(const OpShared &S, const PathConf &pc, bool fwd, int nvar, const int *vars,
-                           int nd, int tid, int nthr, T *W)
+// f32 for the spectra kernels, f64 for the seismograms).  A weight is
+//     as D0(node) + azz D1(node) + af D2(node),
+// D0, D1 the s- and z-derivatives of the node's basis function at the point, D2 its value
+// over s (on the axis its s-derivative), so the 75 values D and the coefficients (as, azz,
+// af) of every (component, variable) are formed once and each weight takes 3 products
+// instead of the terms' table and 10 node sums (k_op_setup, bound by its FP64 operations:
+// 49.7 -> 21.5 ms over 12.2M pairs of 8 x 25 weights).  nthr >= 64; sync orders LDS accesses
+// of the nthr threads.
+template <class T, class SYNC>
+__device__ __forceinline__ void op_weights(OpShared &S, const PathConf &pc, bool fwd, int nvar, const int *vars,
+                                           int nd, int tid, int nthr, T *W, SYNC sync)
 {
+    static_assert(6 * kMaxVar <= 64, "one thread per coefficient");
     const bool axial = S.axial != 0;
-    const int total = nd * nvar * 25;
+    const int ncv = nd * nvar;
     const double *Gx = axial ? c_basis.G1 : c_basis.G2;
-    for (int idx = tid; idx < total; idx += nthr) {
-        int n = idx % 25, v = (idx / 25) % nvar, c = idx / (25 * nvar);
-        int k = n % 5, l = n / 5;
-        int var = vars[v];
+    double as = 0.0, azz = 0.0, af = 0.0;
+    if (tid < ncv) {
+        const int c = tid / nvar, var = vars[tid - c * nvar];
         // simulation of this variable and its local index
         int si, pole, vl;
         if (fwd) {
@@ -1000,31 +1000,43 @@ __device__ void op_weights(const OpShared &S, const PathConf &pc, bool fwd, int 
             tab = pole == 0 ? kTrMono : (pole == 1 ? kTrDi : kTrQuad);
             nt = pole == 0 ? 3 : 4;
         }
-        double as = 0.0, azz = 0.0, af = 0.0;
         for (int q = 0; q < nt; ++q) {
             if (tab[q].var != vl) continue;
             double m = S.M[c][si][pc.full ? tab[q].comp : 0] * (double)tab[q].coef;
             if (tab[q].op == 0) as += m; else if (tab[q].op == 1) azz += m; else af += m;
         }
+    }
+    double d[2] = {0.0, 0.0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int idx = tid + h * nthr;
+        if (idx >= 75) break;
+        const int q = idx / 25, n = idx - 25 * q, k = n % 5, l = n / 5, o = q == 1 ? 2 : 0;
+        // D2 takes of the derivatives only what the axis calls for
+        const bool af2 = q == 2, onax = axial && k == 0;
         double w = 0.0;
-        // xi-derivative part: sum_i Pxi(i, l) * GT(i, k),  GT(i, k) = Gx[k + 5 i]
+        // xi-derivative part: sum_i Lil inv_j(i, l) GT(i, k),  GT(i, k) = Gx[k + 5 i]
         for (int i = 0; i < 5; ++i) {
-            const double *ij = S.invj[i + 5 * l];
-            double Lil = S.li[i] * S.lj[l];
-            double pxi = Lil * (as * ij[0] + azz * ij[2]);
-            if (axial && i == 0) pxi += af * Lil * ij[0];
-            w += pxi * Gx[k + 5 * i];
+            const double x = S.li[i] * S.lj[l] * S.invj[i + 5 * l][o] * Gx[k + 5 * i];
+            if (!af2 || (axial && i == 0)) w += x;
         }
-        // eta-derivative part: sum_j Peta(k, j) * G(l, j),  G(l, j) = G2[l + 5 j]
+        // eta-derivative part: sum_j Lkj inv_j(k, j) G(l, j),  G(l, j) = G2[l + 5 j]
         for (int j = 0; j < 5; ++j) {
-            const double *ij = S.invj[k + 5 * j];
-            double Lkj = S.li[k] * S.lj[j];
-            double peta = Lkj * (as * ij[1] + azz * ij[3]);
-            if (axial && k == 0) peta += af * Lkj * ij[1];
-            w += peta * c_basis.G2[l + 5 * j];
+            const double x = S.li[k] * S.lj[j] * S.invj[k + 5 * j][o + 1] * c_basis.G2[l + 5 * j];
+            if (!af2 || onax) w += x;
         }
-        if (!(axial && k == 0)) w += af * S.li[k] * S.lj[l] * S.sinv[k + 5 * l];
-        W[(c * nvar + v) * 25 + n] = (T)w;
+        if (af2 && !onax) w += S.li[k] * S.lj[l] * S.sinv[n];
+        d[h] = w;
+    }
+    sync();
+    if (tid < ncv) { S.cf[tid][0] = as; S.cf[tid][1] = azz; S.cf[tid][2] = af; }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        if (tid + h * nthr < 75) S.D[0][tid + h * nthr] = d[h];
+    sync();
+    for (int idx = tid; idx < ncv * 25; idx += nthr) {
+        const int cv = idx / 25, n = idx - 25 * cv;
+        W[idx] = (T)(S.cf[cv][0] * S.D[0][n] + S.cf[cv][1] * S.D[1][n] + S.cf[cv][2] * S.D[2][n]);
     }
 }
 
@@ -1032,9 +1044,9 @@ __device__ void build_weights(OpShared &S, const DevDb &db, const PathConf &pc, 
                               const Located &L, bool fwd, int nvar, const int *vars, int nd,
                               const int *comps, bool src_mode)
 {
-    op_setup_parts(S, db, pc, fr, L, fwd, nd, comps, src_mode, threadIdx.x, blockDim.x, 160, 192, 224);
+    op_setup_parts(S, db, pc, fr, L, fwd, nd, comps, src_mode, threadIdx.x, blockDim.x, 160, 192, 200);
     __syncthreads();
-    op_weights(S, pc, fwd, nvar, vars, nd, threadIdx.x, blockDim.x, S.W);
+    op_weights(S, pc, fwd, nvar, vars, nd, threadIdx.x, blockDim.x, S.W, [] { __syncthreads(); });
     __syncthreads();
 }
 
@@ -1067,7 +1079,7 @@ __global__ __launch_bounds__(kStrainThreads) void k_seis(DevDb db, PathConf pc, 
     }
     __syncthreads();
     const int nvar = pc.nvar_bwd;
-    op_weights(S, pc, false, nvar, pc.bwd_vars, 6, tid, kStrainThreads, Wd);
+    op_weights(S, pc, false, nvar, pc.bwd_vars, 6, tid, kStrainThreads, Wd, [] { __syncthreads(); });
     __syncthreads();
     const int nt = pc.nt;
     const size_t blk = (size_t)25 * nt;
@@ -1133,11 +1145,16 @@ __global__ __launch_bounds__(64 * kSetupWaves) void k_op_setup(DevDb db, PathCon
     const int nd = fwd ? pc.nd_f : pc.nd_b;
     const int *comps = fwd ? pc.comps_f : pc.comps_b;
     const int frame = fwd ? 0 : 1 + (q - (q / R) * R);
-    if (live) op_setup_parts(S, db, pc, frames[frame], L, fwd != 0, nd, comps, true, lane, 64, 40, 50, 56);
-    __syncthreads();
+    if (live) op_setup_parts(S, db, pc, frames[frame], L, fwd != 0, nd, comps, true, lane, 64, 40, 50, 0);
+    // a wave's tables are its own
+    const auto sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     if (!live) return;
+    sync();
     const size_t item = fwd ? (size_t)q : (size_t)lb;
-    op_weights(S, pc, fwd != 0, nvar, vars, nd, lane, 64, Wout + item * (size_t)(nd * nvar * 25));
+    op_weights(S, pc, fwd != 0, nvar, vars, nd, lane, 64, Wout + item * (size_t)(nd * nvar * 25), sync);
     if (lane < 36) {
         const int i = lane / 6, c = lane - (lane / 6) * 6;
         Qout[item * 36 + lane] = (pc.full && c < nd) ? S.Q[i][c] : 0.0f;
