@@ -2150,7 +2150,7 @@ int mc_step(State &G, const Task &T, int *nwork_out, std::vector<std::pair<hipEv
     const int ne = T.nelems, P = T.P, R = G.R, nk = G.nk;
     hipStream_t st = G.stream;
     VoxState vs = vox_state(G);
-    hipLaunchKernelGGL(k_step_begin, dim3((ne + 255) / 256), dim3(256), 0, st, ne, nk, G.S.max_iter, vs,
+    hipLaunchKernelGGL(k_step_begin, dim3((ne + kStepWaves - 1) / kStepWaves), dim3(64 * kStepWaves), 0, st, ne, nk, G.S.max_iter, vs,
                        G.live.p, G.working.p);
     HIPCHECK(hipGetLastError());
     hipLaunchKernelGGL(k_compact, dim3(1), dim3(1024), 0, st, ne, G.working.p, G.work_list.p, G.nwork.p);
@@ -2169,7 +2169,8 @@ int mc_step(State &G, const Task &T, int *nwork_out, std::vector<std::pair<hipEv
     int rc;
     for (int w0 = 0; w0 < nwork; w0 += wc)
         if ((rc = eval_chunk(G, P, w0, std::min(wc, nwork - w0), evs))) return rc;
-    hipLaunchKernelGGL(k_mc, dim3(nwork), dim3(256), 0, st, nwork, P, nk, R, G.work_list.p, G.phys.p,
+    // a thread per kernel of the voxel, up to 1024
+    hipLaunchKernelGGL(k_mc, dim3(nwork), dim3(std::min(1024, (nk + 63) / 64 * 64)), 0, st, nwork, P, nk, R, G.work_list.p, G.phys.p,
                        G.nbasis > 1 && !G.vox ? G.bweights.p : nullptr, G.masked.p, G.active.p, G.d_k_rec.p, G.d_k_nbk.p, G.volume.p, G.allowed_var.p,
                        G.S.allowed_relative_error, vs, G.evals.p, G.err.p);
     HIPCHECK(hipGetLastError());
