@@ -512,7 +512,7 @@ typedef struct {
     /* per-launch choice (bwd_path -1): the matrix cores when cost_group_us x groups of   */
     /* 16 pairs + cost_run_us x element runs < cost_pair_us x pairs, else the per-pair    */
     /* kernel; measured by mck_tune (the matrix-core and per-pair kernels' event times),  */
-    /* defaults scaled from c1's at mck_init                                              */
+    /* defaults scaled from c1's at mck_init (with 10 us more on the matrix cores' side)  */
     double  cost_group_us, cost_run_us, cost_pair_us;
     double  auto_ms;           /* best time of the per-launch choice on the points        */
 } mck_tuning_t;

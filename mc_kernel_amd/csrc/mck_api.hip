@@ -410,6 +410,7 @@ struct State {
     // group of 16 pairs and per element run of the matrix-core path, per pair of the
     // per-pair path (set at init from c1's measured costs, measured by mck_tune)
     double cost_group_us = 0.0, cost_run_us = 0.0, cost_pair_us = 0.0;
+    double cost_launch_us = 0.0;                  // added to the matrix cores' side while the costs are the defaults
     int bwd_path_env = -1;                        // MCK_BWD_PATH: 0 per-pair, 1 matrix cores
     int mfma_xcd = 1;                             // MCK_MFMA_XCD: groups in XCD-contiguous ranges
     int mfma_waves = 1;                           // MCK_MFMA_WAVES: waves per element run (1, 2, 4)
@@ -1167,7 +1168,8 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
     HIPCHECK(hipStreamSynchronize(st));
     const int nerun = cnt[0], ngroups = cnt[1];
     // the per-launch choice: the per-pair kernel when it costs less for these pairs
-    if (G.bwd_path_env < 0 && G.cost_pair_us * npairs < G.cost_group_us * ngroups + G.cost_run_us * nerun)
+    if (G.bwd_path_env < 0
+        && G.cost_pair_us * npairs < G.cost_group_us * ngroups + G.cost_run_us * nerun + G.cost_launch_us)
         return launch_status(launch_bwd(G, db, npairs, order, loc_b, Wb, Qb, phys, base_out, active, P));
     G.stats.mfma_runs += nerun;
     const int J = pc.nvar_bwd * 25, KS = mfma_ks(pc.nvar_bwd), NBLK = mfma_nblock(pc.nd_b, pc.nvar_bwd);
@@ -1757,14 +1759,21 @@ int init_impl(const mck_setup_t *s) {
         G.mfma_waves = (w == 2 || w == 4) ? w : 1;
     }
     {
-        // c1 (nt 2048, 4 + 4 components, 2 backward variables): 0.355 us per group, 0.93 us
-        // per element run, 0.0985 us per pair (k_bwd_mfma 22.6 ms / 63,650 groups,
-        // k_elem_spectra 3.0 ms / 3,239 runs, k_bwd_eval 86.2 ms / 875k pairs), scaled
-        // with the trace length and the carried components / traces
+        // c1 (nt 2048, 4 + 4 components, 2 backward variables): 0.31 us per group and 0.46 us
+        // per element run (k_bwd_mfma and k_elem_spectra over 58,355 groups, 31,181 runs of
+        // 32 steps of 100 tets), 0.0985 us per pair (k_bwd_eval 86.2 ms / 875k pairs),
+        // scaled with the trace length and the carried components / traces.  These steps
+        // (16,000 pairs in 1,820 groups each, 9 pairs a group) lie on the matrix cores'
+        // side: 1.09 ms a step against 1.78 in k_bwd_eval; 400 scattered points of 10
+        // receivers (one pair a group) on the other: 2.2 ms against 0.62
         const double sc = G.pc.nt / 2048.0, J = G.pc.nvar_bwd * 25.0, KS = std::ceil(J / 4.0);
-        G.cost_group_us = 0.355 * sc * (KS * G.pc.nd_b) / (13.0 * 4.0) * (0.5 + 0.5 * G.pc.nd_f / 4.0);
-        G.cost_run_us = 0.93 * sc * J / 50.0;
+        G.cost_group_us = 0.31 * sc * (KS * G.pc.nd_b) / (13.0 * 4.0) * (0.5 + 0.5 * G.pc.nd_f / 4.0);
+        G.cost_run_us = 0.46 * sc * J / 50.0;
         G.cost_pair_us = 0.0985 * sc * (G.pc.nd_f + G.pc.nd_b) / 8.0;
+        // two kernels that drain against one: 37 points of 3 receivers (one pair a group,
+        // 6 + 6 components) 97 us against 67 in k_bwd_eval, where the terms above alone
+        // say 75 and 7.4; a launch whose pairs say less than 10 us never goes there
+        G.cost_launch_us = 10.0;
     }
     // tuning knob: points per evaluation launch (smaller launches keep the forward
     // spectra of a launch in the last-level cache)
@@ -2598,6 +2607,7 @@ int mck_set_tuning(const mck_tuning_t *t) {
         G.cost_group_us = t->cost_group_us;
         G.cost_run_us = t->cost_run_us;
         G.cost_pair_us = t->cost_pair_us;
+        G.cost_launch_us = 0.0;
     }
     return MCK_OK;
 }
@@ -2663,6 +2673,7 @@ int mck_tune(int32_t npts, const double *xyz, int32_t reps, mck_tuning_t *out) {
         G.cost_group_us = out->cost_group_us;
         G.cost_run_us = out->cost_run_us;
         G.cost_pair_us = out->cost_pair_us;
+        G.cost_launch_us = 0.0;
         G.bwd_path_env = -1;
         G.mfma_waves = all[bm].waves;
         G.mfma_xcd = all[bm].xcd;
