@@ -421,23 +421,31 @@ __device__ __forceinline__ float mfma_wave_max(float x)
     return __builtin_bit_cast(float, m > n ? m : n);
 }
 
-// max(m, |a|, |b|) in one instruction (fmaxf would quiet NaNs first)
+// (No instruction is written in asm here: the compiler keeps the wait states that matrix and
+// DPP instructions need around the vector instructions it forms itself, not around asm.)
+
+// max(m, |a|, |b|) in one instruction (the IEEE maximum: fmaxf would quiet NaNs first)
 __device__ __forceinline__ float mfma_max3(float m, float a, float b)
 {
-    float r;
-    asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
-    return r;
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, fabsf(a)), fabsf(b));
 }
 
 // x, y (scaled into fp16's range) = hi + lo to 22 bits, as packed halves: fp16 conversion in
-// pairs and the remainders by one mixed-precision FMA each (exact)
-__device__ __forceinline__ void mfma_split2(float x, float y, unsigned &hi, unsigned &lo)
+// pairs and the remainders by one mixed-precision FMA each (exact).  neg: -1 whose value
+// the compiler does not see (mfma_neg_one): x - (float)h would take two instructions.
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float mfma_neg_one()
 {
-    float rx, ry;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(hi) : "v"(x), "v"(y));
-    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(rx) : "v"(hi), "v"(x));
-    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(ry) : "v"(hi), "v"(y));
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(lo) : "v"(rx), "v"(ry));
+    float neg = -1.0f;
+    asm("" : "+s"(neg));
+    return neg;
+}
+__device__ __forceinline__ void mfma_split2(float x, float y, float neg, unsigned &hi, unsigned &lo)
+{
+    const v2h h = __builtin_convertvector((vec2f{x, y}), v2h);
+    const vec2f r = {__builtin_fmaf((float)h[0], neg, x), __builtin_fmaf((float)h[1], neg, y)};
+    hi = __builtin_bit_cast(unsigned, h);
+    lo = __builtin_bit_cast(unsigned, __builtin_convertvector(r, v2h));
 }
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
@@ -515,6 +523,7 @@ __device__ __forceinline__ void mfma_group_setup(MfmaGroup<NDF, NDB> &G, int grp
     int e;
     (void)frexpf(mx, &e);
     G.ew = 14 - e;
+    const float neg = mfma_neg_one();
 #pragma unroll
     for (int b = 0; b < NBLK; ++b) {
         if (NW > 1 && b % NW != wv) continue;
@@ -522,7 +531,7 @@ __device__ __forceinline__ void mfma_group_setup(MfmaGroup<NDF, NDB> &G, int grp
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             unsigned h, o;
-            mfma_split2(ldexpf(w[b][2 * q], G.ew), ldexpf(w[b][2 * q + 1], G.ew), h, o);
+            mfma_split2(ldexpf(w[b][2 * q], G.ew), ldexpf(w[b][2 * q + 1], G.ew), neg, h, o);
             hi[q] = h;
             lo[q] = o;
         }
@@ -714,17 +723,17 @@ __device__ __forceinline__ void mfma_tile(const MfmaGroup<NDF, NDB> &G, MfmaSlot
             a[s].y = ldexpf(a[s].y, eu - 126);
         }
     }
-    const float us = ldexpf(1.0f, min(eu, 126));
+    const float us = ldexpf(1.0f, min(eu, 126)), neg = mfma_neg_one();
 #pragma unroll
     for (int v = 0; v < NVB; ++v) {
         v4u h4[4];                                             // re hi, re lo, im hi, im lo
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             unsigned h, o;
-            mfma_split2(a[8 * v + 2 * q].x * us, a[8 * v + 2 * q + 1].x * us, h, o);
+            mfma_split2(a[8 * v + 2 * q].x * us, a[8 * v + 2 * q + 1].x * us, neg, h, o);
             h4[0][q] = h;
             h4[1][q] = o;
-            mfma_split2(a[8 * v + 2 * q].y * us, a[8 * v + 2 * q + 1].y * us, h, o);
+            mfma_split2(a[8 * v + 2 * q].y * us, a[8 * v + 2 * q + 1].y * us, neg, h, o);
             h4[2][q] = h;
             h4[3][q] = o;
         }
