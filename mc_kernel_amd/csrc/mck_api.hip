@@ -864,12 +864,13 @@ int build_kernels(State &G) {
                 q = e;
             }
             int n = 0;
+            rd.h0 = rd.nslot ? rd.slot_h[0] : 0;               // (slots ordered by window spectrum)
             for (int c = 0; c < 3; ++c) {
                 const int b = n;
                 for (int q = 0; q < rd.nslot; ++q)
                     if ((rd.slot_bk[q] == 0 ? 0 : rd.slot_bk[q] == 1 ? 1 : 2) == c) {
                         rd.cls_pos[q] = n;
-                        rd.cls_h[n++] = rd.slot_h[q];
+                        rd.cls_h[n++] = rd.slot_h[q] - rd.h0;
                     }
                 while ((n - b) & 3) { rd.cls_h[n] = rd.cls_h[b]; ++n; }
                 rd.cls_end[c] = n;

@@ -164,8 +164,11 @@ struct RecDesc {
     // the slots by base-kernel class for the matrix-core kernel: lambda (slot_bk 0), mu
     // (1), combinations; class c holds the positions c ? cls_end[c - 1] : 0 .. cls_end[c] - 1,
     // each class padded to a multiple of 4 positions (groups of 4 matrix-core columns;
-    // padding: another position's window spectrum, a sum nobody reads); cls_h: window
-    // spectrum of a position, cls_pos: position of a slot
+    // padding: another position's window spectrum, a sum nobody reads); cls_pos: position of
+    // a slot; cls_h: window spectrum of a position, counted from the receiver's first, h0
+    // (a receiver's window spectra follow each other: at most kMaxSlots rows, so that
+    // 32-bit offsets from row h0 reach them however large the table is)
+    int h0;
     int cls_h[kMaxSlots + 12];
     int cls_pos[kMaxSlots];
     int cls_end[3];

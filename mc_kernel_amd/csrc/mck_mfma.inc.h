@@ -567,8 +567,8 @@ __device__ __forceinline__ void mfma_group_setup(MfmaGroup<NDF, NDB> &G, int grp
 }
 
 // A wave's window spectra and slot sums: per group of 4 class positions (one class), lane l
-// reads column l % 4's spectrum at the bins of its pair (hoff: bytes to the row and the
-// lane's bins) and holds D[pair][column] (mfma_slot_sum's layout).  The first NG groups'
+// reads column l % 4's spectrum at the bins of its pair (hoff: bytes from the receiver's
+// first row to the row and the lane's bins) and holds D[pair][column] (mfma_slot_sum's layout).  The first NG groups'
 // sums stay in registers across the tiles (NG: 2, 4, 6 or 8, at least the receivers' groups up
 // to 8; groups past a receiver's are summed into values nobody reads), further ones in LDS.
 // The x and y products have a sum each: two chains of dependent products.
@@ -687,14 +687,14 @@ __device__ __forceinline__ void mfma_load_u(const float2 *Ue, const unsigned (&u
 template <int NDF, int NDB, int NVB, int NG, class NextU, class NextF>
 __device__ __forceinline__ void mfma_tile(const MfmaGroup<NDF, NDB> &G, MfmaSlots<NG> &S, float2 (&a)[8 * NVB],
                                           float4 (&f4)[NDF][2], const v8h *sW, double *sAcc, int l, int t,
-                                          const PathConf &pc, const RecDesc &rd, const float2 *Hp, NextU &&next_u,
+                                          const PathConf &pc, const RecDesc &rd, const float2 *Hr, NextU &&next_u,
                                           NextF &&next_f)
 {
     constexpr int KS = 8 * NVB, PF = NG < 4 ? NG : 4;          // window spectra of PF groups loaded ahead
     // Loads complete in the order they are issued, so they are issued in the order of their
     // use: this tile's window spectra, then the next tile's element spectra (when this
     // tile's are split) and forward spectra (when this tile's are multiplied).
-    const float2 *Ht = Hp + (t << 4);
+    const float2 *Ht = Hr + (t << 4);
     float4 h[PF][2];
 #pragma unroll
     for (int g = 0; g < PF; ++g) {
@@ -931,6 +931,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, NDB <= 4 ? 2 : 1) void k_bwd_mfma(
     const int ntile = (pc.nomega + 15) >> 4;
     MfmaSlots<NG> S;
     mfma_slots_init(S, rd, l, pc.fstride);
+    const float2 *Hr = Hp + (size_t)rd.h0 * pc.fstride;
     unsigned uoff[8];
     mfma_uoff(l, uoff);
     // the next tile's element and forward spectra are loaded into the registers of this
@@ -941,7 +942,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, NDB <= 4 ? 2 : 1) void k_bwd_mfma(
     mfma_load_f<NDF>(Fp, l, min(wv, ntile - 1), f4);
     for (int t = wv; t < ntile; t += NW) {
         const int tn = t + NW < ntile ? t + NW : t;
-        mfma_tile<NDF, NDB, NVB, NG>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hp,
+        mfma_tile<NDF, NDB, NVB, NG>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hr,
                                  [&](float2 (&x)[KS]) { mfma_load_u<NVB>(Ue, uoff, tn, x); },
                                  [&](float4 (&x)[NDF][2]) { mfma_load_f<NDF>(Fp, l, tn, x); });
     }
@@ -1009,6 +1010,7 @@ __global__ __launch_bounds__(64 * W) void k_bwd_mfma_wg(
         const float2 *Fp = F + (size_t)(mine ? G.p : 0) * NDF * pc.fstride;
         MfmaSlots<kMfmaMaxRegGroups> S;
         mfma_slots_init(S, rd, l, pc.fstride);
+        const float2 *Hr = Hp + (size_t)rd.h0 * pc.fstride;
         for (int t = 0; t < ntile; ++t) {
             float2 nx[PER];
             const bool more = t + 1 < ntile;
@@ -1026,7 +1028,7 @@ __global__ __launch_bounds__(64 * W) void k_bwd_mfma_wg(
                 for (int s = 0; s < KS; ++s) a[s] = tile[(32 * (s >> 3) + 8 * bq + (s & 7)) * 16 + jp];
                 float4 f4[NDF][2];
                 mfma_load_f<NDF>(Fp, l, t, f4);
-                mfma_tile<NDF, NDB, NVB, kMfmaMaxRegGroups>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hp, [](float2 (&)[KS]) {},
+                mfma_tile<NDF, NDB, NVB, kMfmaMaxRegGroups>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hr, [](float2 (&)[KS]) {},
                                          [](float4 (&)[NDF][2]) {});
             }
             if (more) {
