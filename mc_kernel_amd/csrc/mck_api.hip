@@ -1218,8 +1218,8 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
         if (W > 1 && mfma_wg_lds(KS, NBLK, pc.max_cls, W) > 160 * 1024) W = W > 2 ? 2 : 1;
         if (W > 1 && mfma_wg_lds(KS, NBLK, pc.max_cls, W) > 160 * 1024) W = 1;
         const size_t smem_w = mfma_wg_lds(KS, NBLK, pc.max_cls, W);
-        // slot groups in registers: those of the largest receiver, up to 8
-        const int ng = std::min(kMfmaMaxRegGroups, 2 * ((pc.max_cls / 4 + 1) / 2));
+        // slot groups in registers: those of the largest receiver, up to the form's limit
+        const int ng = std::min(mfma_reg_groups(pc.nd_f, pc.nd_b), 2 * ((pc.max_cls / 4 + 1) / 2));
 #define EVAL1(NF, NB, NV, NG)                                                                     \
         if (ng == NG && pc.nd_f == NF && pc.nd_b == NB && pc.nvar_bwd == NV) {                                \
             if (smem_m > 65536)                                                                   \
@@ -1244,11 +1244,18 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
                                active, P, G.d_rec_r.p);                                           \
             launched = true;                                                                      \
         }
-#define EVAL(NF, NB, NV) \
-        if (W == 1) { EVAL1(NF, NB, NV, 2) EVAL1(NF, NB, NV, 4) EVAL1(NF, NB, NV, 6) EVAL1(NF, NB, NV, 8) }       \
+#define EVAL4(NF, NB, NV) EVAL1(NF, NB, NV, 2) EVAL1(NF, NB, NV, 4)
+#define EVAL6(NF, NB, NV) EVAL4(NF, NB, NV) EVAL1(NF, NB, NV, 6)
+#define EVAL8(NF, NB, NV) EVAL6(NF, NB, NV) EVAL1(NF, NB, NV, 8)
+#define EVAL(NF, NB, NV, LIMIT)                                                                   \
+        static_assert(mfma_reg_groups(NF, NB) == LIMIT, "kernels of every register group count"); \
+        if (W == 1) { EVAL##LIMIT(NF, NB, NV) }                                                   \
         else { EVALW(NF, NB, NV, 2) EVALW(NF, NB, NV, 4) }
-        EVAL(1, 1, 2) EVAL(1, 1, 3) EVAL(4, 4, 2) EVAL(6, 4, 2) EVAL(4, 6, 3) EVAL(6, 6, 3)
+        EVAL(1, 1, 2, 8) EVAL(1, 1, 3, 8) EVAL(4, 4, 2, 6) EVAL(6, 4, 2, 4) EVAL(4, 6, 3, 8) EVAL(6, 6, 3, 8)
 #undef EVAL
+#undef EVAL8
+#undef EVAL6
+#undef EVAL4
 #undef EVALW
 #undef EVAL1
         if (!launched) return fail(MCK_EINVAL, "no matrix-core kernel for these strain components");

@@ -568,11 +568,25 @@ __device__ __forceinline__ void mfma_group_setup(MfmaGroup<NDF, NDB> &G, int grp
 
 // A wave's window spectra and slot sums: per group of 4 class positions (one class), lane l
 // reads column l % 4's spectrum at the bins of its pair (hoff: bytes from the receiver's
-// first row to the row and the lane's bins) and holds D[pair][column] (mfma_slot_sum's layout).  The first NG groups'
-// sums stay in registers across the tiles (NG: 2, 4, 6 or 8, at least the receivers' groups up
-// to 8; groups past a receiver's are summed into values nobody reads), further ones in LDS.
-// The x and y products have a sum each: two chains of dependent products.
+// first row to the row and the lane's bins) and holds D[pair][column] (mfma_slot_sum's
+// layout).  The first NG groups' sums stay in registers across the tiles, further ones in
+// LDS.  NG: that of the receiver with most groups, even, up to mfma_reg_groups; a receiver
+// with fewer leaves the pairs of groups past its own out (of an odd last pair, one is summed
+// into values nobody reads).  The x and y products have a sum each: two chains of dependent
+// products.
 constexpr int kMfmaMaxRegGroups = 8;
+
+// Groups of a form's kernel in registers.  With 4 backward components more than these do not
+// fit the 256 registers of 2 waves a SIMD and spill in every tile, which costs more than
+// sums in LDS: 400 tets, 10 receivers, nt 2048, 16 + 16 slots (8 groups): 9.9 ms with 8
+// groups in registers and 8.1 with 6 (4 forward components), 14.4 and 9.7 with 4 (6 forward
+// components; 12 + 12 slots: 9.6 with 6 groups in registers, 8.3 with 4).  Trace-only
+// kernels keep 8 (3 registers spilled with 3 variables: 12.6 ms at 8 groups against 13.3
+// with 6 in registers), and 6 backward components, at one wave a SIMD, hold 8 as well.
+__host__ __device__ constexpr int mfma_reg_groups(int ndf, int ndb)
+{
+    return ndb == 4 ? (ndf == 6 ? 4 : 6) : kMfmaMaxRegGroups;
+}
 
 template <int NG>
 struct MfmaSlots {
@@ -683,8 +697,9 @@ __device__ __forceinline__ void mfma_load_u(const float2 *Ue, const unsigned (&u
 // as two products); lane l then holds pair l % 16 at bins kb = 16 t + 4 (l / 16) .. + 3 and
 // forms the base kernels with the forward spectra f4 of the pair's point; then the slot
 // sums Re(bk H) with the receiver's window spectra on the FP64 matrix cores.  next_u and
-// next_f load the next tile's spectra into a and f4 once they are used.
-template <int NDF, int NDB, int NVB, int NG, class NextU, class NextF>
+// next_f load the next tile's spectra into a and f4 once they are used.  MORE: receivers may
+// have more than NG groups of slots.
+template <int NDF, int NDB, int NVB, int NG, bool MORE, class NextU, class NextF>
 __device__ __forceinline__ void mfma_tile(const MfmaGroup<NDF, NDB> &G, MfmaSlots<NG> &S, float2 (&a)[8 * NVB],
                                           float4 (&f4)[NDF][2], const v8h *sW, double *sAcc, int l, int t,
                                           const PathConf &pc, const RecDesc &rd, const float2 *Hr, NextU &&next_u,
@@ -804,6 +819,7 @@ __device__ __forceinline__ void mfma_tile(const MfmaGroup<NDF, NDB> &G, MfmaSlot
     mfma_class(bk0, bk1, S.e0 > 0 ? 0 : (S.e1 > 0 ? 1 : 2), ax, ay);
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
+        if (g > 0 && (g & 1) == 0 && g >= S.ng) break;
         if (g > 0 && (g == S.e0 || g == S.e1)) mfma_class(bk0, bk1, g < S.e1 ? 1 : 2, ax, ay);
         const float4 q0 = h[g % PF][0], q1 = h[g % PF][1];
         if (g + PF < NG) {
@@ -813,7 +829,7 @@ __device__ __forceinline__ void mfma_tile(const MfmaGroup<NDF, NDB> &G, MfmaSlot
         }
         mfma_slot_group(ax, ay, q0, q1, S.accx[g], S.accy[g]);
     }
-    if constexpr (NG == kMfmaMaxRegGroups)
+    if constexpr (MORE)
         for (int g = NG; g < S.ng; ++g) {
             const unsigned off = (unsigned)(rd.cls_h[4 * g + (l & 3)] * pc.fstride + 4 * (l >> 4)) * 8u;
             const float4 q0 = gload4_at(Ht, off), q1 = gload4_at(Ht, off + 16u);
@@ -942,7 +958,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, NDB <= 4 ? 2 : 1) void k_bwd_mfma(
     mfma_load_f<NDF>(Fp, l, min(wv, ntile - 1), f4);
     for (int t = wv; t < ntile; t += NW) {
         const int tn = t + NW < ntile ? t + NW : t;
-        mfma_tile<NDF, NDB, NVB, NG>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hr,
+        mfma_tile<NDF, NDB, NVB, NG, NG == mfma_reg_groups(NDF, NDB)>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hr,
                                  [&](float2 (&x)[KS]) { mfma_load_u<NVB>(Ue, uoff, tn, x); },
                                  [&](float4 (&x)[NDF][2]) { mfma_load_f<NDF>(Fp, l, tn, x); });
     }
@@ -1028,7 +1044,7 @@ __global__ __launch_bounds__(64 * W) void k_bwd_mfma_wg(
                 for (int s = 0; s < KS; ++s) a[s] = tile[(32 * (s >> 3) + 8 * bq + (s & 7)) * 16 + jp];
                 float4 f4[NDF][2];
                 mfma_load_f<NDF>(Fp, l, t, f4);
-                mfma_tile<NDF, NDB, NVB, kMfmaMaxRegGroups>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hr, [](float2 (&)[KS]) {},
+                mfma_tile<NDF, NDB, NVB, kMfmaMaxRegGroups, true>(G, S, a, f4, sW, sAcc, l, t, pc, rd, Hr, [](float2 (&)[KS]) {},
                                          [](float4 (&)[NDF][2]) {});
             }
             if (more) {
