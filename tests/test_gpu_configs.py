@@ -71,7 +71,7 @@ def _check_instantiation(stats, spt, nd_f, nd_b):
     assert (stats["spt"], stats["nd_f"], stats["nd_b"]) == (spt, nd_f, nd_b), stats
 
 
-def _pinned_case(p, spt, nd_f, nd_b, npts=4):
+def _pinned_case(p, spt, nd_f, nd_b, npts=4, path=None):
     import mc_kernel_amd as mk
     o, dev = _oracle_on_device_databases(p)
     try:
@@ -82,8 +82,10 @@ def _pinned_case(p, spt, nd_f, nd_b, npts=4):
         try:
             g_b = k.base_kernels(x)
             _check_instantiation(k.stats(), spt, nd_f, nd_b)
+            assert path is None or k.stats()["bwd_path"] == path
             res = k.slave_work(p.verts, p.conn, halton_offsets=ref["offsets"])
             _check_instantiation(res["stats"], spt, nd_f, nd_b)
+            assert path is None or res["stats"]["bwd_path"] == path
         finally:
             k.close()
     finally:
@@ -109,22 +111,25 @@ C1_REDUCED = dict(nelem_target=1000, ntet=3, npoints_per_step=8, max_iter=2, unm
 def test_c1_explosion_z(monkeypatch, waves):
     """c1's kernel set (10 receivers x 4 Gabor x CC/AM x vp/vs) at nt 2048, explosive
     source, Z receivers: 8 samples per thread, 4 and 4 carried components; the
-    matrix-core evaluation with one wave per group and with 2 and 4 waves per element
-    sharing its spectra (MCK_MFMA_WAVES)."""
+    matrix-core evaluation (MCK_BWD_PATH=1: so few points take the per-pair kernel by
+    themselves) with a workgroup per group and with 2 and 4 waves per element sharing its
+    spectra (MCK_MFMA_WAVES)."""
+    monkeypatch.setenv("MCK_BWD_PATH", "1")
     monkeypatch.setenv("MCK_MFMA_WAVES", str(waves))
     p = synth.make_problem("c1", fill=False, **C1_REDUCED)
     assert p.nkernel == 160 and p.nt == 2048
-    _pinned_case(p, 8, 4, 4)
+    _pinned_case(p, 8, 4, 4, path=1)
 
 
 @pytest.mark.parametrize("waves", [1, 2, 4])
 def test_c1_general_moment_tensor_r(monkeypatch, waves):
     """c1's kernel set with a general moment tensor and R receivers: 6 and 6 carried
-    components (all four forward simulations, the PX backward simulation); one, 2 and 4
-    waves per element run."""
+    components (all four forward simulations, the PX backward simulation); the matrix-core
+    evaluation with a workgroup per group and with 2 and 4 waves per element run."""
+    monkeypatch.setenv("MCK_BWD_PATH", "1")
     monkeypatch.setenv("MCK_MFMA_WAVES", str(waves))
     p = synth.make_problem("c1", fill=False, mij=DC, component="R", **C1_REDUCED)
-    _pinned_case(p, 8, 6, 6)
+    _pinned_case(p, 8, 6, 6, path=1)
 
 
 def test_c2_kernel_set_nt2048():
