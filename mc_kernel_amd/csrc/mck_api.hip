@@ -2633,6 +2633,7 @@ int mck_tune(int32_t npts, const double *xyz, int32_t reps, mck_tuning_t *out) {
     cands.push_back(4);
     *out = mck_tuning_t{};
     const int save_path = G.bwd_path_env, save_w = G.mfma_waves, save_x = G.mfma_xcd;
+    const double save_cost[4] = {G.cost_group_us, G.cost_run_us, G.cost_pair_us, G.cost_launch_us};
     std::vector<double> base((size_t)npts * G.nk * 6);
     // best of reps timed runs after an untimed one; the statistics of the timed runs
     auto timed = [&](double *best_ms) -> int {
@@ -2650,6 +2651,10 @@ int mck_tune(int32_t npts, const double *xyz, int32_t reps, mck_tuning_t *out) {
         G.bwd_path_env = save_path;
         G.mfma_waves = save_w;
         G.mfma_xcd = save_x;
+        G.cost_group_us = save_cost[0];
+        G.cost_run_us = save_cost[1];
+        G.cost_pair_us = save_cost[2];
+        G.cost_launch_us = save_cost[3];
         return rc;
     };
     double best = 0.0, best_mfma = 0.0;
