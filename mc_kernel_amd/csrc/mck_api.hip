@@ -1002,13 +1002,21 @@ int spt_for(int nt) {
 unsigned grid_x8(int n) { return 8u * (unsigned)((n + 7) / 8); }
 
 // points xyz[npts] located in the frames frame0 .. frame0 + nframes - 1 (mesh of D): out
-// [npts][nframes]; active (nullable): receivers in use of each voxel (P points)
+// [npts][nframes]; active (nullable): receivers in use of each voxel (P points).  In launches
+// of at most kLocQueries queries (a grid holds fewer than 2^32 threads, kLocLanes a query).
+constexpr long long kLocQueries = 1ll << 28;
 hipError_t launch_locate(State &G, const DbDev &D, int frame0, int nframes, int npts, const double *xyz,
                          const uint8_t *active, int P, Located *out) {
-    const long long lanes = (long long)npts * nframes * kLocLanes;
-    hipLaunchKernelGGL(k_locate, dim3((unsigned)((lanes + 63) / 64)), dim3(64), 0, G.stream, D.d, G.frames.p, frame0,
-                       nframes, npts, xyz, G.S.planet_radius, active, P, G.R, out, G.err.p);
-    return hipGetLastError();
+    const int step = (int)std::min<long long>(npts, std::max<long long>(1, kLocQueries / nframes / P) * P);
+    for (long long p0 = 0; p0 < npts; p0 += step) {
+        const int n = (int)std::min<long long>(step, npts - p0);
+        const long long lanes = (long long)n * nframes * kLocLanes;
+        hipLaunchKernelGGL(k_locate, dim3((unsigned)((lanes + 63) / 64)), dim3(64), 0, G.stream, D.d, G.frames.p,
+                           frame0, nframes, n, xyz + 3 * p0, G.S.planet_radius,
+                           active ? active + (size_t)(p0 / P) * G.R : nullptr, P, G.R, out + p0 * nframes, G.err.p);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
 }
 
 // operator set-up of n points (fwd) or pairs (bwd) in launch order (null = identity)
