@@ -503,7 +503,7 @@ def roofline(steps, config, traffic_path):
         roof["kernels"] = {
             "k_elem_spectra": {"avg_launch_ms": sp_ms / max(mf_launches, 1), "launches": mf_launches},
             "k_bwd_mfma": {"avg_launch_ms": mf_ms / max(mf_launches, 1), "launches": mf_launches,
-                           "waves_per_launch": sum(s[1]["mfma_groups"] for s in steps) / max(mf_launches, 1)},
+                           "groups_per_launch": sum(s[1]["mfma_groups"] for s in steps) / max(mf_launches, 1)},
             "k_fwd_traces+k_fwd_spectra": {"avg_launch_ms": fwd_ms / max(launches, 1), "launches": launches},
             "backward_stage_ms_per_launch": bwd_ms / max(launches, 1)}
     if traffic:
@@ -615,8 +615,8 @@ def self_check_task(p, verts, conn, sample):
             "tolerance": 1e-5}
 
 
-CANDIDATES = ["per-pair FFTs (k_bwd_eval)", "matrix cores, 1 wave per 16 pairs",
-              "matrix cores, 1 wave per 16 pairs, XCD-contiguous groups",
+CANDIDATES = ["per-pair FFTs (k_bwd_eval)", "matrix cores, a workgroup per 16 pairs",
+              "matrix cores, a workgroup per 16 pairs, XCD-contiguous groups",
               "matrix cores, 2 waves per element (spectra in LDS)", "matrix cores, 4 waves per element (spectra in LDS)"]
 CAND_ORDER = [4, 0, 1, 2, 3]          # candidate_ms index of each row above
 

@@ -257,8 +257,10 @@ int mck_slave_work(int32_t elem_type, int32_t nvpe, int32_t nelems, int32_t nbas
 /*
  * The same work unit evaluated the way the reference loop runs it: one element and one
  * MC step at a time, each step a separate sequence of launches over npoints_per_step
- * points.  Same arguments and results as mck_slave_work; used as the one-point-at-a-time
- * comparator for the batched form.
+ * points.  Same arguments and results as mck_slave_work (bit for bit where both forms'
+ * launches take the same backward path, see mck_tuning_t; to the path's tolerance where
+ * a batch takes the matrix cores and a single element's step the per-pair kernel); used as
+ * the one-point-at-a-time comparator for the batched form.
  */
 int mck_slave_work_plain(int32_t elem_type, int32_t nvpe, int32_t nelems, int32_t nbasis,
                          int32_t nvertices, const double *vertices, const int32_t *conn,
@@ -499,7 +501,7 @@ typedef struct {
     int32_t bwd_path;          /* 0 per-pair FFTs (k_bwd_eval), 1 element spectra and the */
                                /* matrix cores (k_elem_spectra + k_bwd_mfma), -1 chosen   */
                                /* per launch by the costs below (the default)             */
-    int32_t mfma_waves;        /* matrix cores: 1 wave per group of 16 pairs, or 2 / 4     */
+    int32_t mfma_waves;        /* matrix cores: 1: a workgroup per group of 16 pairs; 2, 4: */
                                /* waves per element sharing its spectra through LDS        */
     int32_t mfma_xcd;          /* 1: groups in XCD-contiguous ranges                       */
     int32_t ncandidates;       /* candidates timed                                         */
@@ -512,7 +514,8 @@ typedef struct {
     /* per-launch choice (bwd_path -1): the matrix cores when cost_group_us x groups of   */
     /* 16 pairs + cost_run_us x element runs < cost_pair_us x pairs, else the per-pair    */
     /* kernel; measured by mck_tune (the matrix-core and per-pair kernels' event times),  */
-    /* defaults scaled from c1's at mck_init (with 10 us more on the matrix cores' side)  */
+    /* defaults scaled from c1's at mck_init (with 10 us more on the matrix cores' side:  */
+    /* two kernels start and drain there; given or measured costs are taken alone)        */
     double  cost_group_us, cost_run_us, cost_pair_us;
     double  auto_ms;           /* best time of the per-launch choice on the points        */
 } mck_tuning_t;

@@ -408,12 +408,14 @@ struct State {
     std::vector<std::array<hipEvent_t, 3>> kev;
     // per-launch choice of the backward evaluation (bwd_path_env -1): microseconds per
     // group of 16 pairs and per element run of the matrix-core path, per pair of the
-    // per-pair path (set at init from c1's measured costs, measured by mck_tune)
+    // per-pair path (set at init from c1's measured costs, measured by mck_tune).  The two
+    // paths round differently, so that a result depends on the launch it was part of
+    // within the tolerance (the same voxels in a batch and one by one)
     double cost_group_us = 0.0, cost_run_us = 0.0, cost_pair_us = 0.0;
     double cost_launch_us = 0.0;                  // added to the matrix cores' side while the costs are the defaults
     int bwd_path_env = -1;                        // MCK_BWD_PATH: 0 per-pair, 1 matrix cores
     int mfma_xcd = 1;                             // MCK_MFMA_XCD: groups in XCD-contiguous ranges
-    int mfma_waves = 1;                           // MCK_MFMA_WAVES: waves per element run (1, 2, 4)
+    int mfma_waves = 1;                           // MCK_MFMA_WAVES: 1 a workgroup per group, 2 or 4 waves per element run
     size_t uspec_budget = 0;                      // bytes of element spectra per batch
     DBuf<unsigned char> sort_tmp;
     DBuf<double> phys;
@@ -1221,7 +1223,7 @@ int launch_bwd_mfma(State &G, const DevDb &db, int npairs, const int *keys, cons
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipEventRecord(ev[1], st));
         launched = false;
-        // W waves per element run sharing its spectra through LDS, or one wave per group
+        // a workgroup per group (W = 1), or W waves per element run sharing its spectra through LDS
         int W = G.mfma_waves;
         if (W > 1 && mfma_wg_lds(KS, NBLK, pc.max_cls, W) > 160 * 1024) W = W > 2 ? 2 : 1;
         if (W > 1 && mfma_wg_lds(KS, NBLK, pc.max_cls, W) > 160 * 1024) W = 1;
@@ -1781,14 +1783,19 @@ int init_impl(const mck_setup_t *s) {
         // scaled with the trace length and the carried components / traces.  These steps
         // (16,000 pairs in 1,820 groups each, 9 pairs a group) lie on the matrix cores'
         // side: 1.09 ms a step against 1.78 in k_bwd_eval; 400 scattered points of 10
-        // receivers (one pair a group) on the other: 2.2 ms against 0.62
+        // receivers (one pair a group) on the other: 2.2 ms against 0.62.  (KS counts 4
+        // traces a matrix step, as the costs of every set-up have been scaled; the kernel
+        // takes 32 a step and leaves zero blocks out.)
         const double sc = G.pc.nt / 2048.0, J = G.pc.nvar_bwd * 25.0, KS = std::ceil(J / 4.0);
         G.cost_group_us = 0.31 * sc * (KS * G.pc.nd_b) / (13.0 * 4.0) * (0.5 + 0.5 * G.pc.nd_f / 4.0);
         G.cost_run_us = 0.46 * sc * J / 50.0;
         G.cost_pair_us = 0.0985 * sc * (G.pc.nd_f + G.pc.nd_b) / 8.0;
-        // two kernels that drain against one: 37 points of 3 receivers (one pair a group,
-        // 6 + 6 components) 97 us against 67 in k_bwd_eval, where the terms above alone
-        // say 75 and 7.4; a launch whose pairs say less than 10 us never goes there
+        // two kernels that start and drain against one, 11 to 17 us more for launches that fill
+        // the GPU in neither form: 128 pairs of one receiver in 10 groups and 4 runs (trace
+        // only, nt 1024) take 35.9 us on the matrix cores and 22.7 in k_bwd_eval, 512 pairs
+        // 38.1 and 26.9, 192 pairs of 3 receivers (6 + 6 components, nt 1000) 82.0 and 64.9,
+        // where the terms above say 1.2 against 1.6, 2.8 against 6.3 and 11.6 against 13.9;
+        // the next larger ones stay on the matrix cores (1,600 pairs: 40.2 us against 61.5)
         G.cost_launch_us = 10.0;
     }
     // tuning knob: points per evaluation launch (smaller launches keep the forward

@@ -8,7 +8,7 @@
 // padding and the real FFT are linear too (fft.f90:375-413, 546-601), so
 //     B_c(k) = sum_j W_c,j U_j(k),    U_j = rfft(taper . u_j)
 // The nodal spectra U of every backward element a launch touches are computed once
-// (k_elem_spectra, one workgroup per element); the pairs of an element then form their
+// (k_elem_spectra); the pairs of an element then form their
 // spectra as one matrix product [bins x traces] x [traces x pairs] on the matrix cores
 // (fp32 operands as split fp16 products), fused with the frequency-domain contraction of
 // k_bwd_eval: base kernels per bin (kernel.f90:514-570) against the forward spectra of
@@ -909,16 +909,18 @@ __device__ __forceinline__ void mfma_finish(const MfmaGroup<NDF, NDB> &G, int l,
 // are formed: the host sends kernel sets with anisotropic parameters to k_bwd_eval.  Hp:
 // window spectra, rows fstride apart, zero past nomega; F: forward spectra (tile_at), zero
 // past nomega.  xcd: groups in XCD-contiguous ranges (the groups of an element on one XCD).
-// Bound: half by the forward and element spectra, 4 NDF 128-byte lines a pair and 8-bin row
-// (3.7 TB/s at L2 misses over 12,000 tets x 10 receivers), half by the wave's instructions
-// (f16 matrix products 25 %, splitting and slot sums the rest), at the 2 waves a SIMD that
-// 230 registers leave; 3 waves spill and were slower (12.8 against 9.8 ms a launch).  Tiles
-// contiguous in memory, zero (component, variable) blocks left out, and the slot sums on
-// the FP64 matrix units (4 x 4 x 4, a group of 4 slots and 4 bins a product) in place of
-// FP64 vector products: 357 -> 311 ms (12,000 tets, 10 receivers, nt 2048), 124 -> 88 ms
-// (40 voxels, 200 receivers, nt 4096), 428 -> 417 ms (100 tets, 50 receivers, 24 slots a
+// Bound: by the forward and element spectra, 4 NDF 128-byte lines a pair and 8-bin row (76
+// GB read a launch of 20 ms, 3.8 TB/s, over 50,000 tets x 10 receivers), and by the latency
+// of the wave's instructions in between (vector units 39 % and matrix units 17 % busy there:
+// splitting, base kernels and slot sums) at the 2 waves a SIMD that 201 to 256 registers
+// leave (1 with 6 backward components); 3 waves spill and were slower (12.8 against 9.8 ms a
+// launch).  Tiles contiguous in memory, zero (component, variable) blocks left out, and the
+// slot sums on the FP64 matrix units (4 x 4 x 4, a group of 4 slots and 4 bins a product) in
+// place of FP64 vector products: 357 -> 311 ms (12,000 tets, 10 receivers, nt 2048), 124 ->
+// 88 ms (40 voxels, 200 receivers, nt 4096), 428 -> 417 ms (100 tets, 50 receivers, 24 slots a
 // receiver).  Four waves a group against one: 311 against 294, 88 against 89 and 417 against
-// 460 ms (6 register groups of slots spilled).
+// 460 ms (one wave's 6 register groups of slots spilled): four lose 6 % where groups abound
+// and gain where they are few.
 // ------------------------------------------------------------------------------------
 template <int NDF, int NDB, int NVB, int NG>
 __global__ __launch_bounds__(64 * kMfmaWaves, NDB <= 4 ? 2 : 1) void k_bwd_mfma(
