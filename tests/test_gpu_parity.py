@@ -121,6 +121,26 @@ def test_plain_equals_batched(tiny, gpu):
     assert np.array_equal(a["variance"], b["variance"])
 
 
+@pytest.mark.parametrize("path", [0, 1])
+def test_plain_equals_batched_on_one_path(tiny, gpu, path):
+    """The batched and the plain form agree bit for bit where all launches take one backward
+    path (without a choice of the caller a large batch takes the matrix cores and a single
+    element's step the per-pair kernel, which round differently)."""
+    gpu.set_tuning({"bwd_path": path, "mfma_waves": 1, "mfma_xcd": 1})
+    try:
+        gpu.halton_step = 0
+        a = gpu.slave_work(tiny.verts, tiny.conn)
+        assert a["stats"]["bwd_path"] == path
+        gpu.halton_step = 0
+        b = gpu.slave_work(tiny.verts, tiny.conn, plain=True)
+        assert b["stats"]["bwd_path"] == path
+    finally:
+        gpu.set_tuning({"bwd_path": -1, "mfma_waves": 1, "mfma_xcd": 1})
+    assert np.array_equal(a["niterations"], b["niterations"])
+    assert np.array_equal(a["values"], b["values"])
+    assert np.array_equal(a["variance"], b["variance"])
+
+
 def test_slave_work_vertex_basis(tiny, gpu):
     """Basis functions on the tetrahedra's vertices (nbasis 4): one integrator per basis
     function on the same points, values (ne, 4, nk)."""
